@@ -48,7 +48,7 @@ def test_golden_trace_is_current_with_the_reference_build():
     """Where LeanStream's sources are present (not on GPU test machines), the committed fixture
     must still be what the reference runtime prints."""
     ref = ROOT / "oracle" / "_ref" / "runtime_trace_ref"
-    if not Path(os.environ.get("LEANSTREAM_REFERENCE", "/root/reference")).is_dir():
+    if not Path(os.environ.get("LEANSTREAM_REFERENCE", "/root/reference"), "src", "runtime").is_dir():
         pytest.skip("reference sources not present")
     if not ref.is_file():
         subprocess.run(["make", "-s", "-C", str(ROOT / "oracle"), "ref-trace"], check=True, capture_output=True)
