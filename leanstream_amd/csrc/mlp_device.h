@@ -2084,4 +2084,44 @@ __device__ __forceinline__ void mirror_queue(const MlpArgs& a, uint32_t* slot, u
     }
 }
 
+// ---------------------------------------------------------------------------------
+// Launch ends and argument access shared by the kernel files
+// ---------------------------------------------------------------------------------
+// Words of a ring slot a launch uses: the per-unit execution counters (a line per unit from
+// kSyncUnits on) only with the optional execution counts. Clearing the rest cost a layer of
+// 1434 two-neuron groups 4 us: its slot is 367 KB.
+__device__ __forceinline__ uint32_t ring_words_used(const MlpArgs& a) {
+    return a.executions ? a.slot_words : (a.slot_words < kSyncUnits ? a.slot_words : kSyncUnits);
+}
+
+// Completion proof of the split launch sequence, at the end of its last kernel (the
+// reduction): every workgroup counts itself out in two levels -- per group blk % 8, then
+// the last of each group in kSyncExit -- and the very last one stores the sequence.
+__device__ __forceinline__ void finish_launch(const MlpArgs& a, uint32_t* slot) {
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const uint32_t group = blockIdx.x % 8u;
+    const uint32_t members = (gridDim.x + 7u - group) / 8u;
+    const uint32_t groups = gridDim.x < 8u ? gridDim.x : 8u;
+    if (add_agent(slot + kSyncExitGroups + group * kLine, 1u) == members - 1 &&
+        add_agent(slot + kSyncExit, 1u) == groups - 1)
+        __hip_atomic_store(a.done, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The argument blocks, read where this is called. The compiler loads a kernel's arguments
+// at its entry, and the ones it then keeps in vector lanes (more scalars than fit) make the
+// wave wait for those loads there, before anything else is issued. Read through an address
+// the compiler cannot see through, the blocks' loads follow the ones issued before this call.
+template <class P>
+__device__ __forceinline__ const P* late_params_as() {
+#ifdef __HIP_DEVICE_COMPILE__
+    uint64_t p = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
+    asm volatile("" : "+s"(p));
+    // a constant-address-space pointer: the loads through it stay scalar loads
+    return (const P*)reinterpret_cast<const __attribute__((address_space(4))) P*>(p);
+#else
+    return nullptr;
+#endif
+}
+
 }  // namespace lsamd
