@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <algorithm>
 #include "mlp_args.h"
 #include "mlp_launch.h"
 
@@ -30,13 +31,14 @@ namespace lsamd {
 // split order, then the completion word).
 // ---------------------------------------------------------------------------------
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kDenseCols = 256;    // down-projection columns per workgroup: whole 128-byte weight lines
-constexpr int kDenseDnWaves = kDenseCols / 32;   // 32 columns per wave
-constexpr int kDensePitch = 72;    // fp16 per LDS row: 64 neurons + 8 (rows stay 16-byte aligned)
+constexpr int kDenseCols = 128;    // down-projection columns per workgroup: one scale block
+constexpr int kDenseDnWaves = 8;   // down-projection waves per workgroup, sharing a split's steps
+constexpr int kDenseDnWindow = 4;  // down-projection steps (32 neurons) whose loads a wave keeps in flight
+constexpr uint32_t kDenseDnGroups = 256;   // down-projection workgroups: one a CU
 constexpr int kDenseGuWaves = 8;   // gate/up waves per workgroup, each reduces D / 8 columns
-constexpr int kDensePrefetch = 6;  // units whose down-tile loads are in flight per workgroup (9 loads each)
 constexpr int kDenseGuWindow = 3;  // gate/up steps (64 columns) whose weight loads a wave keeps in flight
 
 __device__ __forceinline__ _Float16 bf16_to_f16(uint32_t bits) {
@@ -45,6 +47,25 @@ __device__ __forceinline__ _Float16 bf16_to_f16(uint32_t bits) {
 
 __device__ __forceinline__ f32x16 mfma32(h8 a, h8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4 mfma16(h8 a, h8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// Orders a wave's own LDS accesses across its lanes (the LDS serves a wave's accesses in
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// h rows as the down projection's A fragments: 16-byte piece (32-neuron half, 16 batch rows,
+// lane) of lane l = row % 16 + 16 ((neuron % 32) / 8), eight neurons a piece. Rows >= batch
+// are zero (cleared at bind).
+__device__ __forceinline__ size_t h16_index(uint32_t dest, uint32_t n, uint32_t row) {
+    return ((size_t)((2 * dest + n / 32) * 2 + row / 16) * 64 + row % 16 + 16 * (n % 32 / 8)) * 8 + n % 8;
 }
 
 // Workgroup barrier ordering LDS traffic only. __syncthreads() is a release/acquire at
@@ -131,7 +152,6 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NI <= 8 ? 4 : 2) void dense_gat
     if (NI > 1) issue_x(1, xq[1]);
     const MlpArgs a = late_params_as<DenseGuParams>()->args;
     const Bounds bd = late_params_as<DenseGuParams>()->b;
-    const uint32_t G = a.group_size;
     const Unit u = resolve(a, bd, desc, (int)D);
     f32x16 cg = {}, cu = {};
     if (u.ok) {
@@ -218,7 +238,6 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NI <= 8 ? 4 : 2) void dense_gat
         }
     }
     __syncthreads();
-    const uint32_t hstride = a.slot_capacity * G;
 #pragma unroll
     for (int r = 0; r < 1024 / (64 * kDenseGuWaves); ++r) {
         const uint32_t e = threadIdx.x + 64 * kDenseGuWaves * r, i = e >> 6, l = e & 63;
@@ -233,7 +252,7 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NI <= 8 ? 4 : 2) void dense_gat
             const float g = round_half(gsum);
             const float up = round_half(usum);
             const float sl = round_half(g / (1.0f + __expf(-g)));
-            a.h16[(size_t)tk * hstride + u.dest * G + half * 32 + (l & 31)] =
+            a.h16[h16_index(u.dest, half * 32 + (l & 31), tk)] =
                 __builtin_bit_cast(uint16_t, (_Float16)(sl * up));
         }
     }
@@ -246,128 +265,160 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NI <= 8 ? 4 : 2) void dense_gat
     }
 }
 
-// One unit's share of a down-projection workgroup's loads. Thread t covers rows
-// 4 (t / 32) .. + 3 and columns 8 (t % 32) .. + 7 of the unit's 64 x 256 weight tile: one
-// 4-byte load per row (a wave's 32 lanes read a row's whole 128-byte line), that row's
-// scale for the columns' block, and 8 bytes of the unit's h rows (batch row t / 16,
-// neurons 4 (t % 16) ..).
-struct DenseDnLoad {
-    uint32_t q[4], sb[4];
-    u32x2 hv;
-    bool ok;
+// Down projection. A workgroup takes the 128 columns (64 bytes of every weight row) of one
+// column tile over one split of the units; its eight waves share the split in steps of 32
+// neurons (half a unit), each step a wave's own from its loads to its matrix instructions, so
+// no wave waits for another before the end.
+//
+// In a step lane (q, o) = (l / 16, l % 16) loads the 4-byte word (8 columns 8 o ..) of the
+// eight neuron rows 8 q ... The halves of two rows' words are joined before decoding, so a
+// decoded pair is (neuron n, neuron n + 1) of one column: B fragments of 16x16x32 MFMAs whose
+// column l % 16 is the tile's column 8 (l % 16) + m, m < 8, with no transposition through
+// LDS (the first version's two barriers, 32 KB of LDS writes and as many reads a unit made it
+// 1.5 us a unit, whatever was in flight). A step's 32 row scales (a tile is one scale block)
+// are one load a wave, dealt to the lanes through 64 bytes of its own LDS.
+//
+// The loads of kDenseDnWindow steps are in flight per wave. The eight partial tiles meet in LDS
+// in a fixed order; the split's sum goes to its fp32 partial rows.
+template <int NF>
+struct DenseDnStep {
+    uint32_t q[8];      // eight rows' words
+    uint32_t s;         // the scale of row l % 32
+    u32x4 h[NF];        // A fragments: batch row 16 f + l % 16, neurons 8 q ..
+    uint32_t ok;
 };
 
-// Branch-free, so that the compiler can count the loads in flight and wait for exactly
-// one unit's: a position past the split, and an invalid descriptor, issue the same loads
-// at the first word of the h rows for every lane (one line per instruction instead of a
-// unit's 8 KB tile again; the h rows are not written by this kernel), with ok = false.
-// h rows >= batch are zero (cleared at bind).
-__device__ __forceinline__ void dense_dn_issue_desc(const MlpArgs& a, const Bounds& b, ExecDesc d, bool in, uint32_t c0,
-                                                    DenseDnLoad& L) {
-    const uint32_t D = a.width, G = a.group_size, t = threadIdx.x;
-    const uint32_t nq = t >> 5, o = t & 31, hr = t >> 4, hp = t & 15;
-    const Unit u = resolve(a, b, d, (int)D);
-    L.ok = in && u.ok;   // an invalid descriptor is reported by the gate/up kernel
-    const uint8_t* grp = L.ok ? u.grp : reinterpret_cast<const uint8_t*>(a.h16);
-    const uint16_t* sc = L.ok ? u.sc : a.h16;
-    const uint32_t col = c0 + 8 * o;
-    const uint32_t on = L.ok ? 1u : 0u;   // 0: every lane reads the h rows' first word
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t n = 4 * nq + r;
-        L.q[r] = *reinterpret_cast<const uint32_t*>(grp + on * ((size_t)(n * 3 + 2) * (D / 2) + col / 2));
-        L.sb[r] = sc[on * ((size_t)(n * 3 + 2) * (D / 128) + col / 128)];
-    }
-    L.hv = *reinterpret_cast<const u32x2*>(a.h16 + on * ((size_t)hr * a.slot_capacity * G + u.dest * G + 4 * hp));
+struct DenseDnParams {
+    const ExecDesc* core;
+    uint32_t core_count, width, splits;
+    MlpArgs args;
+    Bounds b;
+};
+static_assert(offsetof(DenseDnParams, args) == 24 && offsetof(DenseDnParams, b) == 24 + sizeof(MlpArgs),
+              "argument segment layout of dense_down_kernel");
+
+__device__ __forceinline__ uint32_t lane_word(uint32_t v, uint32_t lane) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
+}
+__device__ __forceinline__ uint64_t lane_pointer(uint64_t v, uint32_t lane) {
+    return (uint64_t)lane_word((uint32_t)(v >> 32), lane) << 32 | lane_word((uint32_t)v, lane);
 }
 
-__device__ __forceinline__ void dense_dn_issue(const MlpArgs& a, const Bounds& b, uint32_t un, uint32_t u0,
-                                               uint32_t u1, uint32_t c0, DenseDnLoad& L) {
-    const bool in = un < u1;
-    dense_dn_issue_desc(a, b, a.core[in ? un : u0], in, c0, L);
-}
-
-// LDS position (in halves) of the 8-neuron granule gr of tile column col: rows of 64
-// neurons (128 bytes, so every column starts on the same bank), granules XOR-swizzled by
-// (col ^ col >> 3) & 7: eight consecutive columns (the MFMA's 16-byte reads) take eight
-// different granule slots, and so do eight columns 8 apart (the 8-byte writes of one
-// instruction). Swizzling by bits 3..5 alone left the reads of eight consecutive columns on
-// one slot: a third more bank-conflict cycles in the down kernel (SQ_LDS_BANK_CONFLICT).
-__device__ __forceinline__ uint32_t dn_tile_pos(uint32_t col, uint32_t gr) {
-    return col * 64 + 8 * (gr ^ ((col ^ (col >> 3)) & 7));
-}
-
-// Down projection of 256 columns over one split of the units. Per unit the workgroup
-// dequantises the 64 x 256 weight tile into LDS transposed (column-major, 8-neuron
-// granules, so a lane's eight k slots are eight neurons of its column: one 16-byte LDS
-// read) and stages the unit's h rows; wave w then runs four MFMAs for columns
-// 32 w .. 32 w + 31. The loads of the next kDensePrefetch units are in flight while a
-// unit is computed.
-__global__ __launch_bounds__(64 * kDenseDnWaves) void dense_down_kernel(MlpArgs a, Bounds b) {
-    __shared__ alignas(16) _Float16 wl[kDenseCols * 64];
-    __shared__ alignas(16) _Float16 hl[32][kDensePitch];
-    const uint32_t D = a.width;
-    const uint32_t tiles = D / kDenseCols;
-    // XCD-aware order: workgroup blk runs on XCD blk % 8; the tiles of a split go to one
-    // XCD (kDenseSplits is a multiple of 8), so the split's h rows and down-scale lines
-    // are fetched into that XCD's L2 once instead of once per XCD
-    static_assert(kDenseSplits % 8 == 0, "two splits per XCD");
-    const uint32_t xcd = blockIdx.x % 8u, j = blockIdx.x / 8u;
-    const uint32_t split = xcd + 8u * (j / tiles), ct = j % tiles;
-    const uint32_t c0 = ct * kDenseCols;
-    const uint32_t per = (a.core_count + a.dsplits - 1) / a.dsplits;
-    const uint32_t u0 = min(a.core_count, split * per), u1 = min(a.core_count, u0 + per);
-    const uint32_t t = threadIdx.x;
-    const int lane = lane_id();
-    const uint32_t w = wave_id();
-    const uint32_t nq = t >> 5, o = t & 31;    // weight tile: 4-row group, 8-column group
-    const uint32_t hr = t >> 4, hp = t & 15;   // h tile: batch row, 4-neuron part
-    f32x16 acc = {};
-    DenseDnLoad buf[kDensePrefetch];
-    if (u0 < u1) {
+template <int NF>
+__global__ __launch_bounds__(64 * kDenseDnWaves, 2) void dense_down_kernel(const ExecDesc* hot_core,
+                                                                           uint32_t hot_core_count, uint32_t hot_width,
+                                                                           uint32_t hot_splits, MlpArgs args,
+                                                                           Bounds b) {
+    __shared__ alignas(16) float red[kDenseDnWaves][16 * NF][kDenseCols];
+    __shared__ alignas(16) uint16_t ss[kDenseDnWaves][32];
+    const uint32_t D = hot_width, splits = hot_splits;
+    const uint32_t lane = lane_id(), w = wave_id(), q = lane >> 4, o = lane & 15;
+    // XCD-aware order (workgroup blk runs on XCD blk % 8): the two tiles that share the
+    // 128-byte lines of a weight row are neighbours on one XCD, and so, where the splits are a
+    // multiple of 8, are all tiles of a split, which read the same h rows.
+    const uint32_t combo = blockIdx.x % 8u + 8u * (blockIdx.x / 16u);
+    const uint32_t split = combo % splits, tile = 2u * (combo / splits) + (blockIdx.x / 8u & 1u);
+    if (tile >= D / kDenseCols) return;   // the grid is rounded up to whole XCD rows
+    const uint32_t steps = 2 * hot_core_count;   // of 32 neurons
+    const uint32_t s0 = (uint32_t)((uint64_t)steps * split / splits);
+    const uint32_t s1 = (uint32_t)((uint64_t)steps * (split + 1) / splits);
+    const uint32_t mine = s0 + w < s1 ? (s1 - s0 - w + kDenseDnWaves - 1) / kDenseDnWaves : 0u;   // this wave's steps
+    f32x4 acc[NF][8] = {};
+    for (uint32_t k0 = 0; k0 < mine; k0 += 64) {   // lane i holds the addresses of step k0 + i
+        const uint32_t n = min(mine - k0, 64u);
+        const uint32_t my = s0 + w + kDenseDnWaves * (k0 + min(lane, n - 1));
+        const ExecDesc desc = hot_core[my >> 1];
+        const MlpArgs a = late_params_as<DenseDnParams>()->args;
+        const Bounds bd = late_params_as<DenseDnParams>()->b;
+        const Unit u = resolve(a, bd, desc, (int)D);   // an invalid descriptor is reported by the gate/up kernel
+        const bool ok = u.ok && lane < n;
+        // steps past the end and invalid ones load one word of the h rows in every lane
+        const uint64_t pq = reinterpret_cast<uint64_t>(
+            ok ? u.grp + ((size_t)(32 * (my & 1) * 3 + 2) * (D / 2) + tile * (kDenseCols / 2))
+               : reinterpret_cast<const uint8_t*>(a.h16));
+        const uint64_t ps = reinterpret_cast<uint64_t>(
+            ok ? u.sc + ((size_t)(32 * (my & 1) * 3 + 2) * (D / 128) + tile) : a.h16);
+        const uint64_t ph = reinterpret_cast<uint64_t>(a.h16 + (ok ? (size_t)(2 * u.dest + (my & 1)) * 1024 : 0));
+        const uint32_t mask = ok ? ~0u : 0u;
+        const uint32_t vq = 8 * q * (3 * D / 2) + 4 * o;
+        const uint32_t vs = (lane & 31) * (3 * (D / 128)) * 2;
+        auto issue = [&](uint32_t i, DenseDnStep<NF>& L) {
+            const uint32_t at = min(i, 63u);
+            const uint32_t on = i < n ? lane_word(mask, at) : 0u;
+            const auto* rows = glb(reinterpret_cast<const uint8_t*>(lane_pointer(pq, at)));
+            const auto* sc = glb(reinterpret_cast<const uint8_t*>(lane_pointer(ps, at)));
+            const auto* hp = glb(reinterpret_cast<const u32x4*>(lane_pointer(ph, at)));
+            const uint32_t step = on & (3 * D / 2), vo = on & vq;
 #pragma unroll
-        for (int s = 0; s < kDensePrefetch; ++s) dense_dn_issue(a, b, u0 + s, u0, u1, c0, buf[s]);
-        for (uint32_t base = u0; base < u1; base += kDensePrefetch) {
+            for (int r = 0; r < 8; ++r) L.q[r] = *reinterpret_cast<const LS_GLOBAL uint32_t*>(rows + r * step + vo);
+            L.s = *reinterpret_cast<const LS_GLOBAL uint16_t*>(sc + (on & vs));
 #pragma unroll
-            for (int s = 0; s < kDensePrefetch; ++s) {
-                if (buf[s].ok) {   // uniform across the workgroup
-                    // dequantise the four rows (pairs (column k, column k + 4) per row)
-                    h2 v[4][4];
+            for (int f = 0; f < NF; ++f) L.h[f] = hp[on & (64 * f + lane)];
+            L.ok = on;
+        };
+        DenseDnStep<NF> ring[kDenseDnWindow];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const h2 s2 = {half_bits((uint16_t)buf[s].sb[r]), half_bits((uint16_t)buf[s].sb[r])};
-                        dequant8(buf[s].q[r], s2, v[r]);
-                    }
-                    lds_barrier();   // the previous unit's tiles are read
+        for (int s = 0; s < kDenseDnWindow; ++s) issue(s, ring[s]);
+        for (uint32_t base = 0; base < n; base += kDenseDnWindow) {
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) {   // column 8 o + c: rows 4 nq .. 4 nq + 3
-                        const int k = c & 3;
-                        const bool hi = c >= 4;
-                        const h2 r01 = {hi ? v[0][k].y : v[0][k].x, hi ? v[1][k].y : v[1][k].x};
-                        const h2 r23 = {hi ? v[2][k].y : v[2][k].x, hi ? v[3][k].y : v[3][k].x};
-                        const uint32_t col = 8 * o + c;
-                        *reinterpret_cast<u32x2*>(wl + dn_tile_pos(col, nq >> 1) + 4 * (nq & 1)) =
-                            u32x2{__builtin_bit_cast(uint32_t, r01), __builtin_bit_cast(uint32_t, r23)};
-                    }
-                    *reinterpret_cast<u32x2*>(&hl[hr][4 * hp]) = buf[s].hv;
-                    lds_barrier();
-                    const uint32_t col = 32 * w + (lane & 31);
+            for (int s = 0; s < kDenseDnWindow; ++s) {
+                DenseDnStep<NF>& L = ring[s];
+                if (L.ok) {   // wave-uniform
+                    ss[w][lane & 31] = (uint16_t)L.s;
+                    wave_lds_fence();
+                    const u32x4 sv = *reinterpret_cast<const u32x4*>(&ss[w][8 * q]);
+                    wave_lds_fence();
+                    h8 ha[NF];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const uint32_t gr = 2 * j + (lane >> 5);
-                        const h8 ha = *reinterpret_cast<const h8*>(&hl[lane & 31][8 * gr]);
-                        const h8 wb = *reinterpret_cast<const h8*>(wl + dn_tile_pos(col, gr));
-                        acc = mfma32(ha, wb, acc);
+                    for (int f = 0; f < NF; ++f) ha[f] = __builtin_bit_cast(h8, L.h[f]);
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) {   // columns 8 o + 4 half + k
+                        h2 v[4][4];                          // [row pair][k]
+#pragma unroll
+                        for (int p = 0; p < 4; ++p) {
+                            const uint32_t word = __builtin_amdgcn_perm(L.q[2 * p + 1], L.q[2 * p],
+                                                                        half ? 0x07060302u : 0x05040100u);
+                            dequant8(word, as_h2(sv[p]), v[p]);
+                        }
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            h8 wb;
+#pragma unroll
+                            for (int p = 0; p < 4; ++p) {
+                                wb[2 * p] = v[p][k].x;
+                                wb[2 * p + 1] = v[p][k].y;
+                            }
+#pragma unroll
+                            for (int f = 0; f < NF; ++f) acc[f][4 * half + k] = mfma16(ha[f], wb, acc[f][4 * half + k]);
+                        }
                     }
                 }
-                dense_dn_issue(a, b, base + kDensePrefetch + s, u0, u1, c0, buf[s]);
+                issue(base + kDenseDnWindow + s, L);
             }
         }
     }
+    // Row 16 f + 4 q + i, columns 8 o + m: the two float4 of a lane in the two halves of a row
+    // (a wave's 16-byte accesses are then contiguous within 16 lanes).
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const uint32_t tk = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-        if (tk < a.batch) a.dpart[((size_t)split * 32 + tk) * D + c0 + 32 * w + (lane & 31)] = acc[i];
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float* row = red[w][16 * f + 4 * q + i];
+            *reinterpret_cast<f32x4*>(row + 4 * o) = f32x4{acc[f][0][i], acc[f][1][i], acc[f][2][i], acc[f][3][i]};
+            *reinterpret_cast<f32x4*>(row + 64 + 4 * o) = f32x4{acc[f][4][i], acc[f][5][i], acc[f][6][i], acc[f][7][i]};
+        }
+    __syncthreads();
+    const MlpArgs a = late_params_as<DenseDnParams>()->args;
+    constexpr uint32_t kQuads = kDenseCols / 4;
+#pragma unroll
+    for (uint32_t p = 0; p < 16 * NF * kQuads / (64 * kDenseDnWaves); ++p) {
+        const uint32_t e = threadIdx.x + 64 * kDenseDnWaves * p, row = e / kQuads, j = e % kQuads;
+        f32x4 v = {};
+#pragma unroll
+        for (int k = 0; k < kDenseDnWaves; ++k)   // fixed order: deterministic
+            v += *reinterpret_cast<const f32x4*>(&red[k][row][64 * (j & 1) + 4 * (j >> 1)]);
+        if (row < a.batch)
+            *reinterpret_cast<f32x4*>(a.dpart + ((size_t)split * 32 + row) * D + tile * kDenseCols + 4 * j) = v;
     }
 }
 
@@ -431,26 +482,19 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
     const bool mine = idx < hot_batch * W;
     if (mine) {
         const uint32_t tk = idx / W, col = idx - tk * W;
-        if (hot_dsplits == kDenseSplits) {
-            float4 p[kDenseSplits];
+        // every split's load in flight
+        float4 p[kDenseSplits];
 #pragma unroll
-            for (uint32_t s = 0; s < kDenseSplits; ++s) p[s] = parts[(((size_t)s * 32 + tk) * W + col) / 4];
+        for (uint32_t s = 0; s < kDenseSplits; ++s)
+            if (s < hot_dsplits) p[s] = parts[(((size_t)s * 32 + tk) * W + col) / 4];
 #pragma unroll
-            for (uint32_t s = 0; s < kDenseSplits; ++s) {
+        for (uint32_t s = 0; s < kDenseSplits; ++s)
+            if (s < hot_dsplits) {
                 v.x += p[s].x;
                 v.y += p[s].y;
                 v.z += p[s].z;
                 v.w += p[s].w;
             }
-        } else {
-            for (uint32_t s = 0; s < hot_dsplits; ++s) {
-                const float4 q = parts[(((size_t)s * 32 + tk) * W + col) / 4];
-                v.x += q.x;
-                v.y += q.y;
-                v.z += q.z;
-                v.w += q.w;
-            }
-        }
     }
     const MlpArgs a = late_params_as<DenseReduceParams>()->args;
     uint32_t* slot = a.sync + (a.seq & 1) * a.slot_words;
@@ -497,10 +541,16 @@ hipError_t launch_dense(const MlpArgs& args, const Bounds& bounds, hipStream_t s
         void* gargs[] = {&a.core, &cx16, &a, &b};
         if (e == hipSuccess)
             e = hipLaunchKernel(gate_up, dim3(2 * a.core_count), dim3(64 * kDenseGuWaves), gargs, 0, stream);
-        void* dargs[] = {&a, &b};
+        // One workgroup a CU, and no more splits than leave each of its waves a step.
+        const uint32_t tiles = a.width / kDenseCols;
+        a.dsplits = std::min({kDenseSplits, std::max(1u, kDenseDnGroups / tiles),
+                              (2 * a.core_count + kDenseDnWaves - 1) / kDenseDnWaves});
+        const uint32_t combos = a.dsplits * (tiles / 2);
+        void* dargs[] = {&a.core, &a.core_count, &a.width, &a.dsplits, &a, &b};
+        const void* down = a.batch > 16 ? reinterpret_cast<const void*>(&dense_down_kernel<2>)
+                                        : reinterpret_cast<const void*>(&dense_down_kernel<1>);
         if (e == hipSuccess)
-            e = hipLaunchKernel(reinterpret_cast<const void*>(&dense_down_kernel),
-                                dim3(a.width / kDenseCols * a.dsplits), dim3(64 * kDenseDnWaves), dargs, 0, stream);
+            e = hipLaunchKernel(down, dim3((combos + 7) / 8 * 16), dim3(64 * kDenseDnWaves), dargs, 0, stream);
     } else {
         a.dsplits = 0;   // nothing to sum: y = 0
     }
