@@ -16,37 +16,33 @@ namespace lsamd {
 //
 // Per batch row the arithmetic is the batch-1 path's: w = fp16(q * scale) exactly, fp32
 // sums of exact products, fp16 roundings of g, u, silu and h, fp32 sum of h * w_down.
-// The products run on v_mfma_f32_32x32x16_f16: the dequantised weights and h are fp16
+// The products run on v_mfma_f32_16x16x32_f16: the dequantised weights and h are fp16
 // values by definition, and bf16 x converts to fp16 exactly (8 significant bits; only
 // |x| < 2^-17 rounds, by less than 2^-25), so every product is exact in fp32 and only the
-// summation order differs. The 32 MFMA rows are the batch rows (rows >= batch are zero).
+// summation order differs. The 16 MFMA rows are batch rows; 17 .. 32 rows take two MFMAs a
+// weight fragment.
 //
-// MFMA fragment layout (v_mfma_f32_32x32x16_f16, checked on gfx950): lane l holds
-// A[row l % 32][k 8 (l / 32) + i] and B[k 8 (l / 32) + i][col l % 32], i < 8; result
-// element i is C[8 (i / 4) + 4 (l / 32) + i % 4][l % 32]. Which k a slot stands for is
-// free as long as A and B agree, so each lane feeds the MFMA from its own contiguous loads.
+// MFMA fragment layout (v_mfma_f32_16x16x32_f16, checked on gfx950): lane l holds
+// A[row l % 16][k 8 (l / 16) + i] and B[k 8 (l / 16) + i][col l % 16], i < 8; result
+// element i is C[4 (l / 16) + i][l % 16]. Which k a slot stands for is free as long as A and
+// B agree, so each lane feeds the MFMA from its own contiguous loads.
 //
-// Four launches: x conversion (bf16 -> paired fp16, once per layer), gate/up (h rows in
-// fp16), down projection (fp32 partial rows per split of the units), reduction (fixed
-// split order, then the completion word).
+// Three launches: gate/up (h rows in fp16), down projection (fp32 partial rows per split of
+// the units), reduction (fixed split order, then the completion word).
 // ---------------------------------------------------------------------------------
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kDenseCols = 128;    // down-projection columns per workgroup: one scale block
 constexpr int kDenseDnWaves = 8;   // down-projection waves per workgroup, sharing a split's steps
 constexpr int kDenseDnWindow = 4;  // down-projection steps (32 neurons) whose loads a wave keeps in flight
 constexpr uint32_t kDenseDnGroups = 256;   // down-projection workgroups: one a CU
-constexpr int kDenseGuWaves = 8;   // gate/up waves per workgroup, each reduces D / 8 columns
-constexpr int kDenseGuWindow = 3;  // gate/up steps (64 columns) whose weight loads a wave keeps in flight
+constexpr int kDenseGuWaves = 8;   // gate/up waves per workgroup
+constexpr int kDenseGuWindow = 8;  // gate/up steps (8 neurons x 128 columns) whose weight loads a wave keeps in flight
+constexpr uint32_t kDenseGuGroups = 256;   // gate/up workgroups: one a CU
 
 __device__ __forceinline__ _Float16 bf16_to_f16(uint32_t bits) {
     return (_Float16)__builtin_bit_cast(float, bits << 16);
-}
-
-__device__ __forceinline__ f32x16 mfma32(h8 a, h8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
 __device__ __forceinline__ f32x4 mfma16(h8 a, h8 b, f32x4 c) {
@@ -77,191 +73,254 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// x (bf16 [batch][D]) -> x16: fp16 MFMA A fragments in dequant8's pairing. Within each
-// 8-column group the slots hold columns (0, 4, 1, 5, 2, 6, 3, 7), so one 16-byte piece
-// is the A fragment matching a dequantised weight word. The pieces are stored in the
-// order the gate/up waves load them: fragment f = 4 (c / 64) + (c % 32) / 8 holds, for
-// lane l, row l % 32 and columns 64 (c / 64) + 32 (l / 32) + 8 ((c % 32) / 8) .. + 7 at
-// byte 1024 f + 16 l, so every x load of a wave reads one contiguous kilobyte. Rows >=
-// batch are zero. Once per layer, shared by every gate/up workgroup.
-__device__ __forceinline__ uint32_t x16_piece(uint32_t row, uint32_t c) {   // 16-byte piece index
-    const uint32_t f = 4 * (c / 64) + (c % 32) / 8, l = row + 32 * ((c % 64) / 32);
-    return 64 * f + l;
-}
-
-// Its arguments are scalars preloaded into SGPRs: the load goes out at once.
-__global__ __launch_bounds__(kThreads) void dense_x_kernel(const uint16_t* x, uint16_t* x16, uint32_t width,
-                                                           uint32_t batch) {
-    const uint32_t D = width, groups = D / 8;
-    const uint32_t idx = blockIdx.x * kThreads + threadIdx.x;   // row * groups + group
-    const uint32_t row = idx / groups, grp = idx - row * groups;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (row < batch) v = *glb(reinterpret_cast<const u32x4*>(x + (size_t)row * D + 8 * grp));
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+// Eight bf16 columns of x as fp16 in dequant8's pairing: columns (0, 4, 1, 5, 2, 6, 3, 7).
+__device__ __forceinline__ u32x4 x_pairs(u32x4 v) {
     h8 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        o[2 * i] = bf16_to_f16((w[i >> 1] >> (16 * (i & 1))) & 0xffffu);
-        o[2 * i + 1] = bf16_to_f16((w[(i + 4) >> 1] >> (16 * (i & 1))) & 0xffffu);
+        o[2 * i] = bf16_to_f16((v[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+        o[2 * i + 1] = bf16_to_f16((v[(i + 4) >> 1] >> (16 * (i & 1))) & 0xffffu);
     }
-    glb(reinterpret_cast<h8*>(x16))[x16_piece(row, 8 * grp)] = o;
+    return __builtin_bit_cast(u32x4, o);
 }
 
-// Gate/up of one 32-neuron half of one unit for all batch rows. Wave w reduces the
-// eighth [w D/8, (w+1) D/8) of the input in NI steps of 64 columns; the eight partial
-// tiles meet in LDS. Lane l (neuron 32 half + l % 32, row l % 32 of x) takes 32
-// consecutive columns per step: 16 bytes of each weight row and 64 bytes of x16. Up to
-// d = 4096 the kernel stays within 128 registers (four waves per SIMD: two workgroups per
-// CU, so the whole layer's workgroups are resident at once) with the weights of
-// kDenseGuWindow steps in flight per wave.
-// The dense kernels' argument segments (each parameter at its natural alignment): the
-// leading scalars are preloaded into SGPRs, the blocks are read late (late_params_as).
+// NT consecutive scales (2-byte aligned memory) as packed pairs.
+template <int NT>
+__device__ __forceinline__ void load_scales(const LS_GLOBAL uint8_t* p, uint32_t (&out)[(NT + 1) / 2]) {
+    typedef uint32_t any32 __attribute__((aligned(2)));
+    typedef u32x2 any64 __attribute__((aligned(2)));
+    typedef u32x4 any128 __attribute__((aligned(2)));
+    if constexpr (NT == 1) {
+        out[0] = *reinterpret_cast<const LS_GLOBAL uint16_t*>(p);
+    } else if constexpr (NT == 2) {
+        out[0] = *reinterpret_cast<const LS_GLOBAL any32*>(p);
+    } else if constexpr (NT == 4) {
+        const u32x2 v = *reinterpret_cast<const LS_GLOBAL any64*>(p);
+        out[0] = v.x;
+        out[1] = v.y;
+    } else {
+        static_assert(NT == 8, "1, 2, 4 or 8 steps a wave");
+        const u32x4 v = *reinterpret_cast<const LS_GLOBAL any128*>(p);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = v[i];
+    }
+}
+
+__device__ __forceinline__ uint32_t lane_word(uint32_t v, uint32_t lane) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
+}
+__device__ __forceinline__ uint64_t lane_pointer(uint64_t v, uint32_t lane) {
+    return (uint64_t)lane_word((uint32_t)(v >> 32), lane) << 32 | lane_word((uint32_t)v, lane);
+}
+
+// Gate/up. An item is eight neurons of a unit: their gate rows and their up rows are the 16
+// columns of a 16x16x32 MFMA's B operand (lane l % 16: gate of neuron l % 8, then up), so a
+// step of 128 columns is one 16-byte weight load a lane and one decode chain. Items of eight
+// neurons spread a layer over the CUs to within an eighth of a unit.
+//
+// A workgroup is persistent over items wg, wg + groups, ...: KW of its eight waves split D,
+// NT steps each, and a wave holds the x fragments of its columns in registers for all of its
+// items (32 rows x 512 columns are 128 registers at d = 4096). x is read, converted and dealt
+// to the MFMA layout once per workgroup instead of once per 32 neurons (117 MB of L2 reads at
+// 4096 x 224 groups, twice the weights) by a launch of its own. The weight loads of the next
+// kDenseGuWindow steps, whatever item they belong to, are in flight per wave. At the end of an
+// item the waves' partial tiles meet in LDS in a fixed order, one barrier an item.
+//
+// Where the x of 17 .. 32 rows does not fit the registers (d = 8192) a workgroup takes 16 rows
+// (`halves` = 2): workgroups blk and blk + 8, on one XCD, read the same weights.
 struct DenseGuParams {
     const ExecDesc* core;
-    const uint16_t* x16;
+    const uint16_t* x;
+    uint32_t core_count, batch, groups, halves;
     MlpArgs args;
     Bounds b;
 };
-static_assert(offsetof(DenseGuParams, args) == 16 && offsetof(DenseGuParams, b) == 16 + sizeof(MlpArgs),
+static_assert(offsetof(DenseGuParams, args) == 32 && offsetof(DenseGuParams, b) == 32 + sizeof(MlpArgs),
               "argument segment layout of dense_gate_up_kernel");
 
-// The unit's descriptor and the first x16 steps go out from the preloaded arguments; the
-// argument blocks are read behind them.
-template <int NI>
-__global__ __launch_bounds__(64 * kDenseGuWaves, NI <= 8 ? 4 : 2) void dense_gate_up_kernel(
-    const ExecDesc* hot_core, const uint16_t* hot_x16, MlpArgs args, Bounds b) {
-    __shared__ float red[kDenseGuWaves / 2][2][16][64];   // 32 KB: two workgroups per CU fit
-    constexpr uint32_t D = NI * 64 * kDenseGuWaves;
-    constexpr uint32_t kq = D / kDenseGuWaves;
-    const uint32_t unit = blockIdx.x >> 1, half = blockIdx.x & 1;
-    const ExecDesc desc = hot_core[unit];
-    const int lane = lane_id();
-    const uint32_t w = wave_id();
-    const uint32_t n = half * 32 + (lane & 31), hh = lane >> 5, row = lane & 31;
-    // x16 of step t (four 16-byte fragments per lane, each wave-contiguous) is loaded two
-    // steps ahead, from a ring of three; steps 0 and 1 go out before the weights. Loads
-    // complete in issue order, so each step waits only for what it uses.
-    const LS_GLOBAL u32x4* xf = glb(reinterpret_cast<const u32x4*>(hot_x16));
-    u32x4 xq[3][4];
-    auto issue_x = [&](int t, u32x4 (&dst)[4]) {
-        const uint32_t k0 = w * kq + 64 * t + 32 * hh;
+template <int NT, int NF, int KW>
+__global__ __launch_bounds__(64 * kDenseGuWaves, NT * NF <= 2 ? 4 : 2) void dense_gate_up_kernel(
+    const ExecDesc* hot_core, const uint16_t* hot_x, uint32_t hot_core_count, uint32_t hot_batch, uint32_t hot_groups,
+    uint32_t hot_halves, MlpArgs args, Bounds b) {
+    constexpr uint32_t D = KW * NT * 128;
+    constexpr uint32_t IG = kDenseGuWaves / KW;          // items a workgroup computes at a time
+    constexpr int WIN = kDenseGuWindow, IPB = WIN / NT;  // steps, items in flight
+    static_assert(WIN % NT == 0, "whole items in flight");
+    constexpr int TT = NT < 4 ? NT : 4, TC = NT / TT;    // x is dealt TT steps at a time
+    constexpr uint32_t PPR = 16 * TT;                    // 16-byte pieces of a row of it
+    constexpr uint32_t RPI = 64 / PPR, NI = 16 / RPI;    // rows per load instruction, instructions
+    constexpr uint32_t kXVecs = 16 * (PPR + 1);          // rows padded by one piece: 16 rows, 16 bank groups
+    constexpr uint32_t kRedVecs = kDenseGuWaves * NF * 64;   // 16-byte vectors of one item's partial tiles
+    constexpr uint32_t kVecs = kDenseGuWaves * kXVecs > 2 * kRedVecs ? kDenseGuWaves * kXVecs : 2 * kRedVecs;
+    __shared__ u32x4 lds[kVecs];
+    const uint32_t lane = lane_id(), w = wave_id(), kw = w % KW, ig = w / KW;
+    const uint32_t q = lane >> 4, c = lane & 15;
+    const uint32_t half = hot_halves > 1 ? blockIdx.x / 8u & 1u : 0u;
+    const uint32_t wg = hot_halves > 1 ? blockIdx.x % 8u + 8u * (blockIdx.x / 16u) : blockIdx.x;
+    const uint32_t items = 8 * hot_core_count;
+    const uint32_t total = wg * IG < items ? (items / IG - wg + hot_groups - 1) / hot_groups : 0u;
+    if (!total) return;
+    // the first descriptors go out ahead of x, which would otherwise return before them
+    uint32_t n = min(total, 64u);
+    uint32_t item = (wg + hot_groups * min(lane, n - 1)) * IG + ig;
+    ExecDesc desc = hot_core[item >> 3];
+    __builtin_amdgcn_sched_barrier(0);
+    // x: each load of a wave is contiguous in its rows (rows past the batch read the last one:
+    // a row of A only reaches its own row of the result, which nobody reads)
+    u32x4 raw[NF][TC][NI];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dst[j] = xf[x16_piece(row, k0 + 8 * j)];
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int tc = 0; tc < TC; ++tc)
+#pragma unroll
+            for (uint32_t i = 0; i < NI; ++i) {
+                const uint32_t row = min(16 * (f + half) + i * RPI + lane / PPR, hot_batch - 1);
+                raw[f][tc][i] = *glb(reinterpret_cast<const u32x4*>(hot_x + (size_t)row * D + kw * (NT * 128) +
+                                                                    tc * (TT * 128) + 8 * (lane % PPR)));
+            }
+    // A batch of up to 64 items: lane i holds the addresses of item k0 + i.
+    const uint32_t row = (c & 7) * 3 + (c >> 3);
+    const uint32_t vw = row * (D / 2) + kw * (NT * 64) + 16 * q;
+    const uint32_t vs = (row * (D / 128) + kw * NT) * 2;
+    uint32_t dest = 0, mask = 0;
+    uint64_t pw = 0, ps = 0;
+    u32x4 ring[WIN];
+    uint32_t sring[IPB][(NT + 1) / 2];
+    const LS_GLOBAL uint8_t* wp = nullptr;
+    uint32_t von = 0;
+    auto issue = [&](uint32_t i, int t, u32x4& dst, uint32_t (&sc)[(NT + 1) / 2]) {
+        if (t == 0) {
+            const uint32_t at = min(i, 63u);
+            const uint32_t on = lane_word(mask, at) & (i < n ? ~0u : 0u);
+            wp = glb(reinterpret_cast<const uint8_t*>(lane_pointer(pw, at)));
+            von = on & vw;
+            const auto* sp = glb(reinterpret_cast<const uint8_t*>(lane_pointer(ps, at)));
+            load_scales<NT>(sp + (on & vs), sc);
+        }
+        dst = *reinterpret_cast<const LS_GLOBAL u32x4*>(wp + von + 64 * t);
     };
-    issue_x(0, xq[0]);
-    if (NI > 1) issue_x(1, xq[1]);
-    const MlpArgs a = late_params_as<DenseGuParams>()->args;
-    const Bounds bd = late_params_as<DenseGuParams>()->b;
-    const Unit u = resolve(a, bd, desc, (int)D);
-    f32x16 cg = {}, cu = {};
-    if (u.ok) {
-        const uint8_t* wg = u.grp + (size_t)(n * 3) * (D / 2);
-        const uint8_t* wu = wg + D / 2;
-        const uint16_t* sg = u.sc + (size_t)(n * 3) * (D / 128);
-        const uint16_t* su = sg + D / 128;
-        // The weights of WIN steps are in flight: step t's pieces go out into the slot
-        // step t - WIN has just been computed from.
-        constexpr int WIN = NI < kDenseGuWindow ? NI : kDenseGuWindow;
-        u32x4 qg[WIN], qu[WIN];
-        auto issue_w = [&](int t) {
-            const uint32_t k0 = w * kq + 64 * t + 32 * hh;
-            qg[t % WIN] = ld_cached16(wg + k0 / 2);   // a row's 128-byte line serves four steps
-            qu[t % WIN] = ld_cached16(wu + k0 / 2);
-        };
-#pragma unroll
-        for (int t = 0; t < WIN; ++t) issue_w(t);
-        // The wave's K range covers SB consecutive scale blocks of each row (step t uses
-        // block t / 2): one 8-byte load per projection row where SB is a multiple of 4.
-        constexpr int SB = NI >= 2 ? NI / 2 : 1;
-        uint32_t sgv[SB], suv[SB];
-        const uint32_t b0 = NI >= 2 ? w * SB : w / 2;
-        if constexpr (SB % 4 == 0) {
-#pragma unroll
-            for (int i = 0; i < SB; i += 4) {
-                const u32x2 gv = *reinterpret_cast<const u32x2*>(sg + b0 + i);
-                const u32x2 uv = *reinterpret_cast<const u32x2*>(su + b0 + i);
-                sgv[i] = gv.x & 0xffffu; sgv[i + 1] = gv.x >> 16; sgv[i + 2] = gv.y & 0xffffu; sgv[i + 3] = gv.y >> 16;
-                suv[i] = uv.x & 0xffffu; suv[i + 1] = uv.x >> 16; suv[i + 2] = uv.y & 0xffffu; suv[i + 3] = uv.y >> 16;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < SB; ++i) {
-                sgv[i] = sg[b0 + i];
-                suv[i] = su[b0 + i];
-            }
+    auto open = [&](uint32_t k0) {
+        if (k0) {
+            n = min(total - k0, 64u);
+            item = (wg + hot_groups * (k0 + min(lane, n - 1))) * IG + ig;
+            desc = hot_core[item >> 3];
         }
-        // keep every load above ahead of the first MFMA (the scheduler would otherwise
-        // sink them next to their uses, leaving two or three in flight per wave)
         __builtin_amdgcn_sched_barrier(0);
+        const MlpArgs a = late_params_as<DenseGuParams>()->args;
+        const Bounds bd = late_params_as<DenseGuParams>()->b;
+        const Unit u = resolve(a, bd, desc, (int)D);
+        const bool ok = u.ok && lane < n;
+        // items past the end and invalid ones load the first word of x in every lane
+        pw = ok ? reinterpret_cast<uint64_t>(u.grp + (size_t)(item & 7) * (8 * 3 * D / 2))
+                : reinterpret_cast<uint64_t>(hot_x);
+        ps = ok ? reinterpret_cast<uint64_t>(u.sc + (size_t)(item & 7) * (8 * 3 * (D / 128)))
+                : reinterpret_cast<uint64_t>(hot_x);
+        mask = ok ? ~0u : 0u;
+        dest = u.dest;
+        // one lane per item reports it
+        if (half == 0 && kw == 0 && lane < n) {
+            if (!u.ok)
+                __hip_atomic_fetch_or(a.status, kStatusBadDescriptor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            else if (!(item & 7) && a.executions)
+                __hip_atomic_fetch_add(a.executions + u.dest, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
 #pragma unroll
-        for (int t = 0; t < NI; ++t) {
-            if (t + 2 < NI) issue_x(t + 2, xq[(t + 2) % 3]);
+        for (int s = 0; s < WIN; ++s) issue(s / NT, s % NT, ring[s], sring[s / NT]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    open(0);
+    // x: bf16 -> paired fp16 (dequant8's order), dealt through the wave's own LDS
+    h8 xa[NF][NT][4];
+    u32x4* xl = lds + w * kXVecs;
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int tc = 0; tc < TC; ++tc) {
+#pragma unroll
+            for (uint32_t i = 0; i < NI; ++i)
+                xl[(i * RPI + lane / PPR) * (PPR + 1) + lane % PPR] = x_pairs(raw[f][tc][i]);
+            wave_lds_fence();
             __builtin_amdgcn_sched_barrier(0);
-            const int sb = NI >= 2 ? t / 2 : 0;   // constant after unrolling
-            const h2 sg2 = {half_bits((uint16_t)sgv[sb]), half_bits((uint16_t)sgv[sb])};
-            const h2 su2 = {half_bits((uint16_t)suv[sb]), half_bits((uint16_t)suv[sb])};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const h8 xa = __builtin_bit_cast(h8, xq[t % 3][j]);   // paired (dense_x_kernel)
-                h2 wgv[4], wuv[4];
-                dequant8(qg[t % WIN][j], sg2, wgv);   // (column 8 j + i, column 8 j + i + 4)
-                dequant8(qu[t % WIN][j], su2, wuv);
-                h8 bg, bu;
+            for (int t = 0; t < TT; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    bg[2 * i] = wgv[i].x;
-                    bg[2 * i + 1] = wgv[i].y;
-                    bu[2 * i] = wuv[i].x;
-                    bu[2 * i + 1] = wuv[i].y;
+                for (int j = 0; j < 4; ++j)
+                    xa[f][tc * TT + t][j] = __builtin_bit_cast(h8, xl[c * (PPR + 1) + 16 * t + 4 * q + j]);
+            wave_lds_fence();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    uint16_t* const h16 = late_params_as<DenseGuParams>()->args.h16;
+    // Sum of the waves' partial tiles of item k (a lane's slice: row 4 q + i of fragment f, column
+    // c), h from the gate (c < 8) and up (c >= 8) lanes of each neuron.
+    auto finish = [&](uint32_t k, uint32_t buffer) {
+        const float* red = reinterpret_cast<const float*>(lds) + buffer * (kRedVecs * 4) + ig * KW * (NF * 256);
+        const uint32_t on = lane_word(mask, k), at = lane_word(dest, k), tile = lane_word(item & 7, k);
+#pragma unroll
+        for (uint32_t sl = 0; sl < (NF * 4 + KW - 1) / KW; ++sl) {
+            const uint32_t slice = kw + KW * sl;
+            if (slice >= NF * 4) break;
+            float v = 0.f;
+#pragma unroll
+            for (uint32_t k2 = 0; k2 < KW; ++k2) v += red[k2 * (NF * 256) + slice * 64 + lane];   // fixed order
+            const float r = round_half(v);
+            const float up = __int_as_float(
+                __builtin_amdgcn_update_dpp(0, __float_as_int(r), 0x128, 0xF, 0xF, false));   // row_ror:8
+            const float sl1 = round_half(r / (1.0f + __expf(-r)));
+            const uint32_t tk = 16 * (slice / 4 + half) + 4 * q + slice % 4;
+            if (on && c < 8 && tk < hot_batch)
+                h16[h16_index(at, 8 * tile + c, tk)] = __builtin_bit_cast(uint16_t, (_Float16)(sl1 * up));
+        }
+    };
+    uint32_t it = 0;   // items finished: the partial tiles' buffer
+    for (uint32_t k0 = 0;;) {
+        for (uint32_t base = 0;; base += IPB) {
+#pragma unroll
+            for (int m = 0; m < IPB; ++m) {
+                f32x4 acc[NF][2] = {};
+                uint32_t sc[(NT + 1) / 2];
+#pragma unroll
+                for (int i = 0; i < (NT + 1) / 2; ++i) sc[i] = sring[m][i];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    u32x4& word = ring[(m * NT + t) % WIN];
+                    const uint16_t s = (uint16_t)(sc[t / 2] >> (16 * (t & 1)));
+                    const h2 s2 = {half_bits(s), half_bits(s)};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        h2 v[4];
+                        dequant8(word[j], s2, v);   // columns (i, i + 4) of the word's eight
+                        h8 wb;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            wb[2 * i] = v[i].x;
+                            wb[2 * i + 1] = v[i].y;
+                        }
+#pragma unroll
+                        for (int f = 0; f < NF; ++f) acc[f][j & 1] = mfma16(xa[f][t][j], wb, acc[f][j & 1]);
+                    }
+                    issue(base + m + IPB, t, word, sring[m]);
+                    __builtin_amdgcn_sched_barrier(0);   // one step's decode at a time: the x fragments fill the registers
                 }
-                cg = mfma32(xa, bg, cg);
-                cu = mfma32(xa, bu, cu);
+                // Partial tiles alternate between two buffers: this barrier ends item k's
+                // computation, so every wave has read item k - 2's (the buffer written next) and
+                // written item k - 1's (the buffer read next).
+                lds_barrier();
+                float* red = reinterpret_cast<float*>(lds) + (it & 1) * (kRedVecs * 4) + w * (NF * 256);
+#pragma unroll
+                for (int f = 0; f < NF; ++f)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) red[(4 * f + i) * 64 + lane] = acc[f][0][i] + acc[f][1][i];
+                if (base + m) finish(base + m - 1, (it + 1) & 1);
+                ++it;
+                if (base + m + 1 >= n) goto last;   // uniform across the workgroup
             }
-            if (t + WIN < NI) issue_w(t + WIN);
         }
-    }
-    // Fixed-order sum of the eight partial tiles: wave w + 4 into wave w, then waves 0..3.
-    constexpr uint32_t HW = kDenseGuWaves / 2;
-    if (w >= HW) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            red[w - HW][0][i][lane] = cg[i];
-            red[w - HW][1][i][lane] = cu[i];
-        }
-    }
-    __syncthreads();
-    if (w < HW) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            red[w][0][i][lane] += cg[i];
-            red[w][1][i][lane] += cu[i];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 1024 / (64 * kDenseGuWaves); ++r) {
-        const uint32_t e = threadIdx.x + 64 * kDenseGuWaves * r, i = e >> 6, l = e & 63;
-        float gsum = 0.f, usum = 0.f;
-#pragma unroll
-        for (int v = 0; v < (int)HW; ++v) {   // fixed order: deterministic
-            gsum += red[v][0][i][l];
-            usum += red[v][1][i][l];
-        }
-        const uint32_t tk = 8 * (i >> 2) + 4 * (l >> 5) + (i & 3);
-        if (u.ok && tk < a.batch) {
-            const float g = round_half(gsum);
-            const float up = round_half(usum);
-            const float sl = round_half(g / (1.0f + __expf(-g)));
-            a.h16[h16_index(u.dest, half * 32 + (l & 31), tk)] =
-                __builtin_bit_cast(uint16_t, (_Float16)(sl * up));
-        }
-    }
-    if (threadIdx.x == 0) {
-        if (!u.ok) {
-            __hip_atomic_fetch_or(a.status, kStatusBadDescriptor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        } else if (half == 0 && a.executions) {
-            __hip_atomic_fetch_add(a.executions + u.dest, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+    last:
+        lds_barrier();
+        finish(n - 1, (it + 1) & 1);
+        k0 += 64;
+        if (k0 >= total) return;
+        open(k0);
     }
 }
 
@@ -296,13 +355,6 @@ struct DenseDnParams {
 };
 static_assert(offsetof(DenseDnParams, args) == 24 && offsetof(DenseDnParams, b) == 24 + sizeof(MlpArgs),
               "argument segment layout of dense_down_kernel");
-
-__device__ __forceinline__ uint32_t lane_word(uint32_t v, uint32_t lane) {
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
-}
-__device__ __forceinline__ uint64_t lane_pointer(uint64_t v, uint32_t lane) {
-    return (uint64_t)lane_word((uint32_t)(v >> 32), lane) << 32 | lane_word((uint32_t)v, lane);
-}
 
 template <int NF>
 __global__ __launch_bounds__(64 * kDenseDnWaves, 2) void dense_down_kernel(const ExecDesc* hot_core,
@@ -344,7 +396,7 @@ __global__ __launch_bounds__(64 * kDenseDnWaves, 2) void dense_down_kernel(const
         const uint32_t vs = (lane & 31) * (3 * (D / 128)) * 2;
         auto issue = [&](uint32_t i, DenseDnStep<NF>& L) {
             const uint32_t at = min(i, 63u);
-            const uint32_t on = i < n ? lane_word(mask, at) : 0u;
+            const uint32_t on = lane_word(mask, at) & (i < n ? ~0u : 0u);
             const auto* rows = glb(reinterpret_cast<const uint8_t*>(lane_pointer(pq, at)));
             const auto* sc = glb(reinterpret_cast<const uint8_t*>(lane_pointer(ps, at)));
             const auto* hp = glb(reinterpret_cast<const u32x4*>(lane_pointer(ph, at)));
@@ -510,37 +562,46 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
 }
 
 namespace {
-const void* dense_gate_up_for(uint32_t width) {
+// Gate/up kernels by width and rows: D = 128 x steps x waves an item is split over.
+struct DenseGu {
+    const void* fn;
+    uint32_t items;    // items a workgroup computes at a time
+    uint32_t halves;   // workgroups the rows of an item are split over
+};
+template <int NT, int NF, int KW>
+DenseGu dense_gu(uint32_t halves = 1) {
+    return {reinterpret_cast<const void*>(&dense_gate_up_kernel<NT, NF, KW>), (uint32_t)(kDenseGuWaves / KW), halves};
+}
+DenseGu dense_gate_up_for(uint32_t width, uint32_t batch) {
+    const bool two = batch > 16;
     switch (width) {
-        case 512: return reinterpret_cast<const void*>(&dense_gate_up_kernel<1>);
-        case 1024: return reinterpret_cast<const void*>(&dense_gate_up_kernel<2>);
-        case 2048: return reinterpret_cast<const void*>(&dense_gate_up_kernel<4>);
-        case 4096: return reinterpret_cast<const void*>(&dense_gate_up_kernel<8>);
-        case 8192: return reinterpret_cast<const void*>(&dense_gate_up_kernel<16>);
-        default: return nullptr;
+        case 512: return two ? dense_gu<1, 2, 4>() : dense_gu<1, 1, 4>();
+        case 1024: return two ? dense_gu<1, 2, 8>() : dense_gu<1, 1, 8>();
+        case 2048: return two ? dense_gu<2, 2, 8>() : dense_gu<2, 1, 8>();
+        case 4096: return two ? dense_gu<4, 2, 8>() : dense_gu<4, 1, 8>();
+        case 8192: return dense_gu<8, 1, 8>(two ? 2 : 1);
+        default: return {nullptr, 0, 0};
     }
 }
 }  // namespace
 
-bool dense_available(int width) { return width > 0 && dense_gate_up_for((uint32_t)width) != nullptr; }
+bool dense_available(int width) { return width > 0 && dense_gate_up_for((uint32_t)width, 1).fn != nullptr; }
 
 hipError_t launch_dense(const MlpArgs& args, const Bounds& bounds, hipStream_t stream) {
     MlpArgs a = args;
     Bounds b = bounds;
-    const void* gate_up = dense_gate_up_for(a.width);
-    if (a.group_size != 64 || !gate_up || a.batch <= kMaxBatch || a.batch > kMaxDenseBatch || !a.dsplits ||
-        !a.h16 || !a.dpart || !a.x16)
+    const DenseGu gu = dense_gate_up_for(a.width, a.batch);
+    if (a.group_size != 64 || !gu.fn || a.batch <= kMaxBatch || a.batch > kMaxDenseBatch || !a.dsplits ||
+        !a.h16 || !a.dpart)
         return hipErrorInvalidValue;
     hipError_t e = hipSuccess;
     if (a.core_count) {
-        uint16_t* x16 = a.x16;
-        void* xargs[] = {&a.x, &x16, &a.width, &a.batch};
-        e = hipLaunchKernel(reinterpret_cast<const void*>(&dense_x_kernel), dim3(32 * a.width / 8 / kThreads),
-                            dim3(kThreads), xargs, 0, stream);
-        const uint16_t* cx16 = a.x16;
-        void* gargs[] = {&a.core, &cx16, &a, &b};
-        if (e == hipSuccess)
-            e = hipLaunchKernel(gate_up, dim3(2 * a.core_count), dim3(64 * kDenseGuWaves), gargs, 0, stream);
+        // groups of workgroups over the items; whole rows of XCDs where the batch is split
+        uint32_t groups = std::min(kDenseGuGroups / gu.halves, 8 * a.core_count / gu.items);
+        if (gu.halves > 1) groups = (groups + 7) / 8 * 8;
+        uint32_t halves = gu.halves;
+        void* gargs[] = {&a.core, &a.x, &a.core_count, &a.batch, &groups, &halves, &a, &b};
+        e = hipLaunchKernel(gu.fn, dim3(groups * halves), dim3(64 * kDenseGuWaves), gargs, 0, stream);
         // One workgroup a CU, and no more splits than leave each of its waves a step.
         const uint32_t tiles = a.width / kDenseCols;
         a.dsplits = std::min({kDenseSplits, std::max(1u, kDenseDnGroups / tiles),

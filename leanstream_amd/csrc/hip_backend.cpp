@@ -24,7 +24,6 @@ struct HipBackend::Impl {
     void* owned_hidden = nullptr;
     uint16_t* h16 = nullptr;     // dense path: fp16 h rows
     float* dpart = nullptr;      // dense path: down-projection partial rows
-    uint16_t* x16 = nullptr;     // dense path: x converted to paired fp16
     bool dense = false;          // batch > kMaxBatch: every launch takes the matrix-core path
     uint32_t* done = nullptr;    // host-coherent: sequence of the last finished launch
     uint32_t* arrivals = nullptr;  // epilogue row workgroups that finished (zero between launches)
@@ -57,7 +56,6 @@ struct HipBackend::Impl {
         if (owned_hidden) (void)hipFree(owned_hidden);
         if (h16) (void)hipFree(h16);
         if (dpart) (void)hipFree(dpart);
-        if (x16) (void)hipFree(x16);
         if (status) (void)hipHostFree(status);
         if (done) (void)hipHostFree(done);
         if (arrivals) (void)hipFree(arrivals);
@@ -82,7 +80,6 @@ struct HipBackend::Impl {
         owned_hidden = nullptr;
         h16 = nullptr;
         dpart = nullptr;
-        x16 = nullptr;
         status = nullptr;
         done = nullptr;
         bound = false;
@@ -120,7 +117,6 @@ int HipBackend::bind(const HipLayerBuffers& b) {
         e = hipMalloc(&p.h16, sizeof(uint16_t) * 32 * b.slot_capacity * b.group_size);
     if (e == hipSuccess && dense)
         e = hipMalloc(&p.dpart, sizeof(float) * lsamd::kDenseSplits * 32 * b.width);
-    if (e == hipSuccess && dense) e = hipMalloc(&p.x16, sizeof(uint16_t) * 32 * b.width);
     // h rows >= batch stay zero: the dense down projection reads all 32 rows
     if (e == hipSuccess && dense) e = hipMemset(p.h16, 0, sizeof(uint16_t) * 32 * b.slot_capacity * b.group_size);
     if (e == hipSuccess)
@@ -193,7 +189,6 @@ int HipBackend::bind(const HipLayerBuffers& b) {
     a.slot_capacity = b.slot_capacity;
     a.h16 = p.h16;
     a.dpart = p.dpart;
-    a.x16 = p.x16;
     a.dsplits = dense ? lsamd::kDenseSplits : 0u;
     p.bounds = {b.cache_groups, b.staging_groups, b.physical_groups};
     slices_ = b.width / lsamd::kDnCols;

@@ -49,7 +49,7 @@ constexpr uint32_t kAccStride = 1;
 constexpr uint32_t kDnCols = 256;  // columns of one down-projection item (two scale blocks)
 constexpr uint32_t kMaxBatch = 4;  // batch rows of one launch (x of every row is kept in LDS)
 constexpr uint32_t kMaxDenseBatch = 32;   // batch rows of the dense (matrix-core) path
-constexpr uint32_t kDenseSplits = 16;     // unit splits of its down projection
+constexpr uint32_t kDenseSplits = 16;     // most unit splits of its down projection
 
 constexpr uint32_t pack_epoch(uint32_t state, uint32_t path, uint32_t total) { return state | (path << 2) | (total << 4); }
 
@@ -212,9 +212,8 @@ struct MlpArgs {
     uint32_t grid;                // workgroups of a persistent launch (workers + the mirror)
     uint32_t pack;                // units per down item: 64 / G for the packed kernels, else 1 (set per launch)
     // dense path (batch > kMaxBatch): x is bf16 [batch][d]
-    uint16_t* h16;                // fp16 h rows [32][slot_capacity * G]
+    uint16_t* h16;                // fp16 h of 32 rows x slot_capacity * G neurons, as MFMA A fragments
     float* dpart;                 // fp32 down-projection partial rows [dsplits][32][d]
-    uint16_t* x16;                // x as fp16 MFMA A fragments, 32 rows x d (dense_x_kernel; rows >= batch zero)
     uint32_t dsplits;
     uint64_t spin_limit;          // bounded waits, in 100 MHz ticks
     // the layer's epilogue, run by the fused launch's last workgroup once every worker is out
