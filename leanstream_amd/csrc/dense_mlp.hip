@@ -4,6 +4,7 @@
 #include <stddef.h>
 #include <stdint.h>
 #include <algorithm>
+#include <type_traits>
 #include "mlp_args.h"
 #include "mlp_launch.h"
 
@@ -31,19 +32,14 @@ namespace lsamd {
 // the units), reduction (fixed split order, then the completion word).
 // ---------------------------------------------------------------------------------
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kDenseCols = 128;    // down-projection columns per workgroup: one scale block
-constexpr int kDenseDnWaves = 8;   // down-projection waves per workgroup, sharing a split's steps
-constexpr int kDenseDnWindow = 4;  // down-projection steps (32 neurons) whose loads a wave keeps in flight
+constexpr int kDenseCols = 256;    // down-projection columns per workgroup: whole 128-byte weight lines
+constexpr int kDenseDnWaves = 8;   // down-projection waves per workgroup: four pairs
 constexpr uint32_t kDenseDnGroups = 256;   // down-projection workgroups: one a CU
 constexpr int kDenseGuWaves = 8;   // gate/up waves per workgroup
-constexpr int kDenseGuWindow = 8;  // gate/up steps (8 neurons x 128 columns) whose weight loads a wave keeps in flight
 constexpr uint32_t kDenseGuGroups = 256;   // gate/up workgroups: one a CU
-
-__device__ __forceinline__ _Float16 bf16_to_f16(uint32_t bits) {
-    return (_Float16)__builtin_bit_cast(float, bits << 16);
-}
 
 __device__ __forceinline__ f32x4 mfma16(h8 a, h8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -73,15 +69,25 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// A buffer of `bytes` bytes at a wave-uniform address. A load past its end returns zero and
+// reads no memory: loads of steps past the end of a wave's work are issued (so that the
+// compiler can count the loads in flight) with bytes = 0. Sent to one word that every wave
+// reads instead, they queued at one L2 channel.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t wave_buffer(uint64_t address, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(address), 0, (int)bytes, 0x00027000);
+}
+
 // Eight bf16 columns of x as fp16 in dequant8's pairing: columns (0, 4, 1, 5, 2, 6, 3, 7).
 __device__ __forceinline__ u32x4 x_pairs(u32x4 v) {
-    h8 o;
+    u32x4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        o[2 * i] = bf16_to_f16((v[i >> 1] >> (16 * (i & 1))) & 0xffffu);
-        o[2 * i + 1] = bf16_to_f16((v[(i + 4) >> 1] >> (16 * (i & 1))) & 0xffffu);
+        const uint32_t a = v[i >> 1], b = v[2 + (i >> 1)];
+        const f32x2 f = {__uint_as_float(i & 1 ? a & 0xffff0000u : a << 16),
+                         __uint_as_float(i & 1 ? b & 0xffff0000u : b << 16)};
+        o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, h2));   // round to nearest even
     }
-    return __builtin_bit_cast(u32x4, o);
+    return o;
 }
 
 // NT consecutive scales (2-byte aligned memory) as packed pairs.
@@ -122,9 +128,12 @@ __device__ __forceinline__ uint64_t lane_pointer(uint64_t v, uint32_t lane) {
 // NT steps each, and a wave holds the x fragments of its columns in registers for all of its
 // items (32 rows x 512 columns are 128 registers at d = 4096). x is read, converted and dealt
 // to the MFMA layout once per workgroup instead of once per 32 neurons (117 MB of L2 reads at
-// 4096 x 224 groups, twice the weights) by a launch of its own. The weight loads of the next
-// kDenseGuWindow steps, whatever item they belong to, are in flight per wave. At the end of an
-// item the waves' partial tiles meet in LDS in a fixed order, one barrier an item.
+// 4096 x 224 groups, twice the weights) by a launch of its own. The weight loads of the
+// next round (two items; one at d >= 4096, whose items are four steps and more) are in flight
+// while a round is computed. At the end of a round the waves' partial tiles meet in LDS in a
+// fixed order, one barrier a round: two items a round and no loads past the end took the kernel
+// from 7.1 to 5.9 us at 2048 columns x 128 groups x 7 rows; at 4096 x 224 x 32 one item a round
+// is the better (17.6 us, two 18.5).
 //
 // Where the x of 17 .. 32 rows does not fit the registers (d = 8192) a workgroup takes 16 rows
 // (`halves` = 2): workgroups blk and blk + 8, on one XCD, read the same weights.
@@ -144,13 +153,12 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NT * NF <= 2 ? 4 : 2) void dens
     uint32_t hot_halves, MlpArgs args, Bounds b) {
     constexpr uint32_t D = KW * NT * 128;
     constexpr uint32_t IG = kDenseGuWaves / KW;          // items a workgroup computes at a time
-    constexpr int WIN = kDenseGuWindow, IPB = WIN / NT;  // steps, items in flight
-    static_assert(WIN % NT == 0, "whole items in flight");
+    constexpr int IPB = NT < 4 ? 2 : 1, WIN = IPB * NT;  // items of a round, their steps
     constexpr int TT = NT < 4 ? NT : 4, TC = NT / TT;    // x is dealt TT steps at a time
     constexpr uint32_t PPR = 16 * TT;                    // 16-byte pieces of a row of it
     constexpr uint32_t RPI = 64 / PPR, NI = 16 / RPI;    // rows per load instruction, instructions
     constexpr uint32_t kXVecs = 16 * (PPR + 1);          // rows padded by one piece: 16 rows, 16 bank groups
-    constexpr uint32_t kRedVecs = kDenseGuWaves * NF * 64;   // 16-byte vectors of one item's partial tiles
+    constexpr uint32_t kRedVecs = IPB * kDenseGuWaves * NF * 64;   // 16-byte vectors of a round's partial tiles
     constexpr uint32_t kVecs = kDenseGuWaves * kXVecs > 2 * kRedVecs ? kDenseGuWaves * kXVecs : 2 * kRedVecs;
     __shared__ u32x4 lds[kVecs];
     const uint32_t lane = lane_id(), w = wave_id(), kw = w % KW, ig = w / KW;
@@ -160,13 +168,13 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NT * NF <= 2 ? 4 : 2) void dens
     const uint32_t items = 8 * hot_core_count;
     const uint32_t total = wg * IG < items ? (items / IG - wg + hot_groups - 1) / hot_groups : 0u;
     if (!total) return;
-    // the first descriptors go out ahead of x, which would otherwise return before them
     uint32_t n = min(total, 64u);
     uint32_t item = (wg + hot_groups * min(lane, n - 1)) * IG + ig;
     ExecDesc desc = hot_core[item >> 3];
     __builtin_amdgcn_sched_barrier(0);
-    // x: each load of a wave is contiguous in its rows (rows past the batch read the last one:
-    // a row of A only reaches its own row of the result, which nobody reads)
+    // x: each load of a wave is contiguous in its rows (rows past the batch read the last one: a row
+    // of A only reaches its own row of the result, which nobody reads). Behind the first weights
+    // instead, x waited for them: 0.7 us more at 4096 columns x 32 rows.
     u32x4 raw[NF][TC][NI];
 #pragma unroll
     for (int f = 0; f < NF; ++f)
@@ -186,18 +194,15 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NT * NF <= 2 ? 4 : 2) void dens
     uint64_t pw = 0, ps = 0;
     u32x4 ring[WIN];
     uint32_t sring[IPB][(NT + 1) / 2];
-    const LS_GLOBAL uint8_t* wp = nullptr;
-    uint32_t von = 0;
+    __amdgpu_buffer_rsrc_t wp = wave_buffer(0, 0);
     auto issue = [&](uint32_t i, int t, u32x4& dst, uint32_t (&sc)[(NT + 1) / 2]) {
         if (t == 0) {
-            const uint32_t at = min(i, 63u);
-            const uint32_t on = lane_word(mask, at) & (i < n ? ~0u : 0u);
-            wp = glb(reinterpret_cast<const uint8_t*>(lane_pointer(pw, at)));
-            von = on & vw;
-            const auto* sp = glb(reinterpret_cast<const uint8_t*>(lane_pointer(ps, at)));
-            load_scales<NT>(sp + (on & vs), sc);
+            const uint32_t at = min(i, n - 1);
+            wp = wave_buffer(lane_pointer(pw, at), i < n ? lane_word(mask, at) & (8 * 3 * D / 2) : 0u);
+            // past the end: the last item's scales again
+            load_scales<NT>(glb(reinterpret_cast<const uint8_t*>(lane_pointer(ps, at))) + (lane_word(mask, at) & vs), sc);
         }
-        dst = *reinterpret_cast<const LS_GLOBAL u32x4*>(wp + von + 64 * t);
+        dst = __builtin_amdgcn_raw_buffer_load_b128(wp, vw, 64 * t, 0);
     };
     auto open = [&](uint32_t k0) {
         if (k0) {
@@ -209,10 +214,9 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NT * NF <= 2 ? 4 : 2) void dens
         const MlpArgs a = late_params_as<DenseGuParams>()->args;
         const Bounds bd = late_params_as<DenseGuParams>()->b;
         const Unit u = resolve(a, bd, desc, (int)D);
-        const bool ok = u.ok && lane < n;
-        // items past the end and invalid ones load the first word of x in every lane
-        pw = ok ? reinterpret_cast<uint64_t>(u.grp + (size_t)(item & 7) * (8 * 3 * D / 2))
-                : reinterpret_cast<uint64_t>(hot_x);
+        const bool ok = u.ok;
+        // an invalid item loads no weights, and its scales from the first words of x
+        pw = reinterpret_cast<uint64_t>(u.grp + (size_t)(item & 7) * (8 * 3 * D / 2));
         ps = ok ? reinterpret_cast<uint64_t>(u.sc + (size_t)(item & 7) * (8 * 3 * (D / 128)))
                 : reinterpret_cast<uint64_t>(hot_x);
         mask = ok ? ~0u : 0u;
@@ -250,39 +254,41 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NT * NF <= 2 ? 4 : 2) void dens
             __builtin_amdgcn_sched_barrier(0);
         }
     uint16_t* const h16 = late_params_as<DenseGuParams>()->args.h16;
-    // Sum of the waves' partial tiles of item k (a lane's slice: row 4 q + i of fragment f, column
-    // c), h from the gate (c < 8) and up (c >= 8) lanes of each neuron.
-    auto finish = [&](uint32_t k, uint32_t buffer) {
-        const float* red = reinterpret_cast<const float*>(lds) + buffer * (kRedVecs * 4) + ig * KW * (NF * 256);
-        const uint32_t on = lane_word(mask, k), at = lane_word(dest, k), tile = lane_word(item & 7, k);
+    // Sum of the waves' partial tiles of the round's items (a lane's slice: row 4 q + i of fragment f,
+    // column c), h from the gate (c < 8) and up (c >= 8) lanes of each neuron.
+    auto finish = [&](uint32_t base, uint32_t buffer) {
+        constexpr uint32_t kSlices = IPB * NF * 4;
+        const float* red = reinterpret_cast<const float*>(lds) + buffer * (kRedVecs * 4) + ig * KW * (IPB * NF * 256);
 #pragma unroll
-        for (uint32_t sl = 0; sl < (NF * 4 + KW - 1) / KW; ++sl) {
+        for (uint32_t sl = 0; sl < (kSlices + KW - 1) / KW; ++sl) {
             const uint32_t slice = kw + KW * sl;
-            if (slice >= NF * 4) break;
+            const uint32_t k = base + slice / (NF * 4), fi = slice % (NF * 4);
+            if (slice >= kSlices || k >= n) break;   // wave-uniform
+            const uint32_t on = lane_word(mask, k), at = lane_word(dest, k), tile = lane_word(item & 7, k);
             float v = 0.f;
 #pragma unroll
-            for (uint32_t k2 = 0; k2 < KW; ++k2) v += red[k2 * (NF * 256) + slice * 64 + lane];   // fixed order
+            for (uint32_t k2 = 0; k2 < KW; ++k2) v += red[k2 * (IPB * NF * 256) + slice * 64 + lane];   // fixed order
             const float r = round_half(v);
-            const float up = __int_as_float(
-                __builtin_amdgcn_update_dpp(0, __float_as_int(r), 0x128, 0xF, 0xF, false));   // row_ror:8
+            const float up =
+                __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(r), 0x128, 0xF, 0xF, false));   // row_ror:8
             const float sl1 = round_half(r / (1.0f + __expf(-r)));
-            const uint32_t tk = 16 * (slice / 4 + half) + 4 * q + slice % 4;
+            const uint32_t tk = 16 * (fi / 4 + half) + 4 * q + fi % 4;
             if (on && c < 8 && tk < hot_batch)
                 h16[h16_index(at, 8 * tile + c, tk)] = __builtin_bit_cast(uint16_t, (_Float16)(sl1 * up));
         }
     };
-    uint32_t it = 0;   // items finished: the partial tiles' buffer
+    uint32_t rounds = 0;   // rounds computed: the partial tiles' buffer
     for (uint32_t k0 = 0;;) {
-        for (uint32_t base = 0;; base += IPB) {
+        auto round = [&](uint32_t base, auto more) {
+            f32x4 acc[IPB][NF][2] = {};
 #pragma unroll
             for (int m = 0; m < IPB; ++m) {
-                f32x4 acc[NF][2] = {};
                 uint32_t sc[(NT + 1) / 2];
 #pragma unroll
                 for (int i = 0; i < (NT + 1) / 2; ++i) sc[i] = sring[m][i];
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    u32x4& word = ring[(m * NT + t) % WIN];
+                    u32x4& word = ring[m * NT + t];
                     const uint16_t s = (uint16_t)(sc[t / 2] >> (16 * (t & 1)));
                     const h2 s2 = {half_bits(s), half_bits(s)};
 #pragma unroll
@@ -296,54 +302,65 @@ __global__ __launch_bounds__(64 * kDenseGuWaves, NT * NF <= 2 ? 4 : 2) void dens
                             wb[2 * i + 1] = v[i].y;
                         }
 #pragma unroll
-                        for (int f = 0; f < NF; ++f) acc[f][j & 1] = mfma16(xa[f][t][j], wb, acc[f][j & 1]);
+                        for (int f = 0; f < NF; ++f) acc[m][f][j & 1] = mfma16(xa[f][t][j], wb, acc[m][f][j & 1]);
                     }
-                    issue(base + m + IPB, t, word, sring[m]);
+                    if constexpr (decltype(more)::value) issue(base + m + IPB, t, word, sring[m]);
                     __builtin_amdgcn_sched_barrier(0);   // one step's decode at a time: the x fragments fill the registers
                 }
-                // Partial tiles alternate between two buffers: this barrier ends item k's
-                // computation, so every wave has read item k - 2's (the buffer written next) and
-                // written item k - 1's (the buffer read next).
-                lds_barrier();
-                float* red = reinterpret_cast<float*>(lds) + (it & 1) * (kRedVecs * 4) + w * (NF * 256);
+                // a last round of one item leaves the second one out
+                if (!decltype(more)::value && base + m + 1 >= n) break;
+            }
+            // Partial tiles alternate between two buffers: this barrier ends the round's
+            // computation, so every wave has read the round before last (the buffer written
+            // next) and written the last one (the buffer read next).
+            lds_barrier();
+            float* red = reinterpret_cast<float*>(lds) + (rounds & 1) * (kRedVecs * 4) + w * (IPB * NF * 256);
+#pragma unroll
+            for (int m = 0; m < IPB; ++m)
 #pragma unroll
                 for (int f = 0; f < NF; ++f)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) red[(4 * f + i) * 64 + lane] = acc[f][0][i] + acc[f][1][i];
-                if (base + m) finish(base + m - 1, (it + 1) & 1);
-                ++it;
-                if (base + m + 1 >= n) goto last;   // uniform across the workgroup
-            }
-        }
-    last:
+                    for (int i = 0; i < 4; ++i) red[((m * NF + f) * 4 + i) * 64 + lane] = acc[m][f][0][i] + acc[m][f][1][i];
+            ++rounds;
+            if (base) finish(base - IPB, rounds & 1);
+        };
+        // the last round requests nothing: a load past the end costs its issue, if no memory
+        uint32_t base = 0;
+        for (; base + IPB < n; base += IPB) round(base, std::true_type{});
+        round(base, std::false_type{});
         lds_barrier();
-        finish(n - 1, (it + 1) & 1);
+        finish(base, (rounds & 1) ^ 1);
         k0 += 64;
         if (k0 >= total) return;
         open(k0);
     }
 }
 
-// Down projection. A workgroup takes the 128 columns (64 bytes of every weight row) of one
-// column tile over one split of the units; its eight waves share the split in steps of 32
-// neurons (half a unit), each step a wave's own from its loads to its matrix instructions, so
-// no wave waits for another before the end.
+// Down projection. A workgroup takes 256 columns (whole 128-byte lines of the weight rows) over
+// one split of the units, in steps of 32 neurons (half a unit). Its waves are four pairs: the
+// pairs share the split's steps, and the two waves of a pair take 128 columns (a scale block)
+// each of the same step, so a step's weight lines, h and scale lines come to the CU once. No
+// wave waits for another before the end.
 //
 // In a step lane (q, o) = (l / 16, l % 16) loads the 4-byte word (8 columns 8 o ..) of the
 // eight neuron rows 8 q ... The halves of two rows' words are joined before decoding, so a
 // decoded pair is (neuron n, neuron n + 1) of one column: B fragments of 16x16x32 MFMAs whose
 // column l % 16 is the tile's column 8 (l % 16) + m, m < 8, with no transposition through
 // LDS (the first version's two barriers, 32 KB of LDS writes and as many reads a unit made it
-// 1.5 us a unit, whatever was in flight). A step's 32 row scales (a tile is one scale block)
-// are one load a wave, dealt to the lanes through 64 bytes of its own LDS.
+// 1.5 us a unit, whatever was in flight). A step's 32 row scales are one load a wave, dealt to
+// the lanes through 64 bytes of its own LDS.
 //
-// The loads of kDenseDnWindow steps are in flight per wave. The eight partial tiles meet in LDS
-// in a fixed order; the split's sum goes to its fp32 partial rows.
+// A step's loads are in flight while the step before it is computed; more of them in flight
+// made the kernel slower (two steps 12.4, three 13.2 us at 4096 columns x 224 groups x 32 rows
+// against 11.3 with none ahead): a load costs its issue, and the ones past the end of a wave's
+// steps are wasted. The partial tiles meet in LDS in a fixed order; the split's sum goes to its
+// fp32 partial rows. Twice the columns a wave (8-byte loads, half the loads a byte) made twice
+// the partial tiles: equal.
 template <int NF>
 struct DenseDnStep {
-    uint32_t q[8];      // eight rows' words
-    uint32_t s;         // the scale of row l % 32
-    u32x4 h[NF];        // A fragments: batch row 16 f + l % 16, neurons 8 q ..
+    uint32_t q[8];   // eight rows' words
+    uint32_t s;      // the scale of row l % 32
+    u32x4 h[NF];     // A fragments: batch row 16 f + l % 16, neurons 8 q ..
     uint32_t ok;
 };
 
@@ -361,114 +378,108 @@ __global__ __launch_bounds__(64 * kDenseDnWaves, 2) void dense_down_kernel(const
                                                                            uint32_t hot_core_count, uint32_t hot_width,
                                                                            uint32_t hot_splits, MlpArgs args,
                                                                            Bounds b) {
-    __shared__ alignas(16) float red[kDenseDnWaves][16 * NF][kDenseCols];
+    constexpr uint32_t kHalf = kDenseCols / 2, kPairs = kDenseDnWaves / 2;
+    __shared__ alignas(16) float red[kDenseDnWaves][16 * NF][kHalf];
     __shared__ alignas(16) uint16_t ss[kDenseDnWaves][32];
     const uint32_t D = hot_width, splits = hot_splits;
     const uint32_t lane = lane_id(), w = wave_id(), q = lane >> 4, o = lane & 15;
-    // XCD-aware order (workgroup blk runs on XCD blk % 8): the two tiles that share the
-    // 128-byte lines of a weight row are neighbours on one XCD, and so, where the splits are a
-    // multiple of 8, are all tiles of a split, which read the same h rows.
-    const uint32_t combo = blockIdx.x % 8u + 8u * (blockIdx.x / 16u);
-    const uint32_t split = combo % splits, tile = 2u * (combo / splits) + (blockIdx.x / 8u & 1u);
-    if (tile >= D / kDenseCols) return;   // the grid is rounded up to whole XCD rows
+    // XCD-aware order (workgroup blk runs on XCD blk % 8): consecutive splits go to consecutive
+    // XCDs, so with 8 or 16 splits all tiles of a split, which read the same h rows and scale
+    // lines, share an L2.
+    const uint32_t split = blockIdx.x % splits, tile = blockIdx.x / splits;
+    const uint32_t half = w & 1, pair = w >> 1;
     const uint32_t steps = 2 * hot_core_count;   // of 32 neurons
     const uint32_t s0 = (uint32_t)((uint64_t)steps * split / splits);
     const uint32_t s1 = (uint32_t)((uint64_t)steps * (split + 1) / splits);
-    const uint32_t mine = s0 + w < s1 ? (s1 - s0 - w + kDenseDnWaves - 1) / kDenseDnWaves : 0u;   // this wave's steps
+    const uint32_t mine = s0 + pair < s1 ? (s1 - s0 - pair + kPairs - 1) / kPairs : 0u;   // this wave's steps
     f32x4 acc[NF][8] = {};
     for (uint32_t k0 = 0; k0 < mine; k0 += 64) {   // lane i holds the addresses of step k0 + i
         const uint32_t n = min(mine - k0, 64u);
-        const uint32_t my = s0 + w + kDenseDnWaves * (k0 + min(lane, n - 1));
+        const uint32_t my = s0 + pair + kPairs * (k0 + min(lane, n - 1));
         const ExecDesc desc = hot_core[my >> 1];
         const MlpArgs a = late_params_as<DenseDnParams>()->args;
         const Bounds bd = late_params_as<DenseDnParams>()->b;
         const Unit u = resolve(a, bd, desc, (int)D);   // an invalid descriptor is reported by the gate/up kernel
-        const bool ok = u.ok && lane < n;
-        // steps past the end and invalid ones load one word of the h rows in every lane
-        const uint64_t pq = reinterpret_cast<uint64_t>(
-            ok ? u.grp + ((size_t)(32 * (my & 1) * 3 + 2) * (D / 2) + tile * (kDenseCols / 2))
-               : reinterpret_cast<const uint8_t*>(a.h16));
-        const uint64_t ps = reinterpret_cast<uint64_t>(
-            ok ? u.sc + ((size_t)(32 * (my & 1) * 3 + 2) * (D / 128) + tile) : a.h16);
-        const uint64_t ph = reinterpret_cast<uint64_t>(a.h16 + (ok ? (size_t)(2 * u.dest + (my & 1)) * 1024 : 0));
-        const uint32_t mask = ok ? ~0u : 0u;
+        // an invalid step loads nothing (its addresses are those of slot, row and destination 0)
+        const uint32_t mask = u.ok ? ~0u : 0u;
+        const uint64_t pq = reinterpret_cast<uint64_t>(u.grp) + (size_t)(32 * (my & 1) * 3 + 2) * (D / 2) +
+                            tile * (kDenseCols / 2) + half * (kHalf / 2);
+        const uint64_t ps = reinterpret_cast<uint64_t>(u.sc + (size_t)(32 * (my & 1) * 3 + 2) * (D / 128) + 2 * tile + half);
+        const uint64_t ph = reinterpret_cast<uint64_t>(a.h16 + (size_t)(2 * u.dest + (my & 1)) * 1024);
         const uint32_t vq = 8 * q * (3 * D / 2) + 4 * o;
         const uint32_t vs = (lane & 31) * (3 * (D / 128)) * 2;
         auto issue = [&](uint32_t i, DenseDnStep<NF>& L) {
-            const uint32_t at = min(i, 63u);
-            const uint32_t on = lane_word(mask, at) & (i < n ? ~0u : 0u);
-            const auto* rows = glb(reinterpret_cast<const uint8_t*>(lane_pointer(pq, at)));
-            const auto* sc = glb(reinterpret_cast<const uint8_t*>(lane_pointer(ps, at)));
-            const auto* hp = glb(reinterpret_cast<const u32x4*>(lane_pointer(ph, at)));
-            const uint32_t step = on & (3 * D / 2), vo = on & vq;
+            L.ok = lane_word(mask, i);
+            const __amdgpu_buffer_rsrc_t rows = wave_buffer(lane_pointer(pq, i), L.ok & (31 * (3 * D / 2) + kHalf / 2));
+            const __amdgpu_buffer_rsrc_t hp = wave_buffer(lane_pointer(ph, i), L.ok & 2048u);
 #pragma unroll
-            for (int r = 0; r < 8; ++r) L.q[r] = *reinterpret_cast<const LS_GLOBAL uint32_t*>(rows + r * step + vo);
-            L.s = *reinterpret_cast<const LS_GLOBAL uint16_t*>(sc + (on & vs));
+            for (int r = 0; r < 8; ++r) L.q[r] = __builtin_amdgcn_raw_buffer_load_b32(rows, vq, r * (3 * D / 2), 0);
+            L.s = *reinterpret_cast<const LS_GLOBAL uint16_t*>(glb(reinterpret_cast<const uint8_t*>(lane_pointer(ps, i))) + vs);
 #pragma unroll
-            for (int f = 0; f < NF; ++f) L.h[f] = hp[on & (64 * f + lane)];
-            L.ok = on;
+            for (int f = 0; f < NF; ++f) L.h[f] = __builtin_amdgcn_raw_buffer_load_b128(hp, 16 * lane, 1024 * f, 0);
         };
-        DenseDnStep<NF> ring[kDenseDnWindow];
+        auto compute = [&](const DenseDnStep<NF>& L) {
+            if (!L.ok) return;   // wave-uniform
+            ss[w][lane & 31] = (uint16_t)L.s;
+            wave_lds_fence();
+            const u32x4 sv = *reinterpret_cast<const u32x4*>(&ss[w][8 * q]);
+            wave_lds_fence();
+            h8 ha[NF];
 #pragma unroll
-        for (int s = 0; s < kDenseDnWindow; ++s) issue(s, ring[s]);
-        for (uint32_t base = 0; base < n; base += kDenseDnWindow) {
+            for (int f = 0; f < NF; ++f) ha[f] = __builtin_bit_cast(h8, L.h[f]);
 #pragma unroll
-            for (int s = 0; s < kDenseDnWindow; ++s) {
-                DenseDnStep<NF>& L = ring[s];
-                if (L.ok) {   // wave-uniform
-                    ss[w][lane & 31] = (uint16_t)L.s;
-                    wave_lds_fence();
-                    const u32x4 sv = *reinterpret_cast<const u32x4*>(&ss[w][8 * q]);
-                    wave_lds_fence();
-                    h8 ha[NF];
+            for (int part = 0; part < 2; ++part) {   // columns 8 o + 4 part + k
+                h2 v[4][4];                          // [row pair][k]
 #pragma unroll
-                    for (int f = 0; f < NF; ++f) ha[f] = __builtin_bit_cast(h8, L.h[f]);
-#pragma unroll
-                    for (int half = 0; half < 2; ++half) {   // columns 8 o + 4 half + k
-                        h2 v[4][4];                          // [row pair][k]
-#pragma unroll
-                        for (int p = 0; p < 4; ++p) {
-                            const uint32_t word = __builtin_amdgcn_perm(L.q[2 * p + 1], L.q[2 * p],
-                                                                        half ? 0x07060302u : 0x05040100u);
-                            dequant8(word, as_h2(sv[p]), v[p]);
-                        }
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            h8 wb;
-#pragma unroll
-                            for (int p = 0; p < 4; ++p) {
-                                wb[2 * p] = v[p][k].x;
-                                wb[2 * p + 1] = v[p][k].y;
-                            }
-#pragma unroll
-                            for (int f = 0; f < NF; ++f) acc[f][4 * half + k] = mfma16(ha[f], wb, acc[f][4 * half + k]);
-                        }
-                    }
+                for (int p = 0; p < 4; ++p) {
+                    const uint32_t word = __builtin_amdgcn_perm(L.q[2 * p + 1], L.q[2 * p],
+                                                                part ? 0x07060302u : 0x05040100u);
+                    dequant8(word, as_h2(sv[p]), v[p]);
                 }
-                issue(base + kDenseDnWindow + s, L);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    h8 wb;
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        wb[2 * p] = v[p][k].x;
+                        wb[2 * p + 1] = v[p][k].y;
+                    }
+#pragma unroll
+                    for (int f = 0; f < NF; ++f) acc[f][4 * part + k] = mfma16(ha[f], wb, acc[f][4 * part + k]);
+                }
             }
+        };
+        DenseDnStep<NF> cur, next;
+        issue(0, cur);
+#pragma unroll 1
+        for (uint32_t i = 1; i < n; ++i) {
+            issue(i, next);
+            compute(cur);
+            cur = next;
         }
+        compute(cur);
     }
-    // Row 16 f + 4 q + i, columns 8 o + m: the two float4 of a lane in the two halves of a row
-    // (a wave's 16-byte accesses are then contiguous within 16 lanes).
+    // Row 16 f + 4 q + i, columns 8 o + m: a lane's two float4 in the two halves of a row (a
+    // wave's 16-byte accesses are then contiguous within 16 lanes).
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float* row = red[w][16 * f + 4 * q + i];
-            *reinterpret_cast<f32x4*>(row + 4 * o) = f32x4{acc[f][0][i], acc[f][1][i], acc[f][2][i], acc[f][3][i]};
-            *reinterpret_cast<f32x4*>(row + 64 + 4 * o) = f32x4{acc[f][4][i], acc[f][5][i], acc[f][6][i], acc[f][7][i]};
-        }
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int part = 0; part < 2; ++part)
+                *reinterpret_cast<f32x4*>(&red[w][16 * f + 4 * q + i][64 * part + 4 * o]) =
+                    f32x4{acc[f][4 * part][i], acc[f][4 * part + 1][i], acc[f][4 * part + 2][i], acc[f][4 * part + 3][i]};
     __syncthreads();
     const MlpArgs a = late_params_as<DenseDnParams>()->args;
     constexpr uint32_t kQuads = kDenseCols / 4;
 #pragma unroll
     for (uint32_t p = 0; p < 16 * NF * kQuads / (64 * kDenseDnWaves); ++p) {
         const uint32_t e = threadIdx.x + 64 * kDenseDnWaves * p, row = e / kQuads, j = e % kQuads;
+        const uint32_t hj = j / (kHalf / 4), jj = j % (kHalf / 4);   // column half, float4 of it
         f32x4 v = {};
 #pragma unroll
-        for (int k = 0; k < kDenseDnWaves; ++k)   // fixed order: deterministic
-            v += *reinterpret_cast<const f32x4*>(&red[k][row][64 * (j & 1) + 4 * (j >> 1)]);
+        for (uint32_t k = 0; k < kPairs; ++k)   // fixed order: deterministic
+            v += *reinterpret_cast<const f32x4*>(&red[2 * k + hj][row][64 * (jj & 1) + 4 * (jj >> 1)]);
         if (row < a.batch)
             *reinterpret_cast<f32x4*>(a.dpart + ((size_t)split * 32 + row) * D + tile * kDenseCols + 4 * j) = v;
     }
@@ -602,16 +613,15 @@ hipError_t launch_dense(const MlpArgs& args, const Bounds& bounds, hipStream_t s
         uint32_t halves = gu.halves;
         void* gargs[] = {&a.core, &a.x, &a.core_count, &a.batch, &groups, &halves, &a, &b};
         e = hipLaunchKernel(gu.fn, dim3(groups * halves), dim3(64 * kDenseGuWaves), gargs, 0, stream);
-        // One workgroup a CU, and no more splits than leave each of its waves a step.
+        // One workgroup a CU, and no more splits than leave each pair of its waves a step.
         const uint32_t tiles = a.width / kDenseCols;
         a.dsplits = std::min({kDenseSplits, std::max(1u, kDenseDnGroups / tiles),
-                              (2 * a.core_count + kDenseDnWaves - 1) / kDenseDnWaves});
-        const uint32_t combos = a.dsplits * (tiles / 2);
+                              (2 * a.core_count + kDenseDnWaves / 2 - 1) / (kDenseDnWaves / 2)});
         void* dargs[] = {&a.core, &a.core_count, &a.width, &a.dsplits, &a, &b};
         const void* down = a.batch > 16 ? reinterpret_cast<const void*>(&dense_down_kernel<2>)
                                         : reinterpret_cast<const void*>(&dense_down_kernel<1>);
         if (e == hipSuccess)
-            e = hipLaunchKernel(down, dim3((combos + 7) / 8 * 16), dim3(64 * kDenseDnWaves), dargs, 0, stream);
+            e = hipLaunchKernel(down, dim3(tiles * a.dsplits), dim3(64 * kDenseDnWaves), dargs, 0, stream);
     } else {
         a.dsplits = 0;   // nothing to sum: y = 0
     }
