@@ -33,7 +33,6 @@ namespace lsamd {
 // ---------------------------------------------------------------------------------
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDenseCols = 256;    // down-projection columns per workgroup: whole 128-byte weight lines
 constexpr int kDenseDnWaves = 8;   // down-projection waves per workgroup: four pairs

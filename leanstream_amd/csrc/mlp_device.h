@@ -12,6 +12,8 @@
 namespace lsamd {
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -127,6 +129,22 @@ __device__ __forceinline__ void dequant8(uint32_t word, h2 s, h2 out[4]) {
 }
 
 __device__ __forceinline__ float dot2(h2 a, h2 b, float c) { return __builtin_amdgcn_fdot2(a, b, c, false); }
+
+// Products on the matrix cores (v_mfma_f32_4x4x4_16b_f16): sixteen independent 4x4 products of
+// depth 4, one per four lanes. Lane l passes A[row l % 4][k] and B[k][column l % 4], k < 4, and
+// receives column l % 4 of the result, element i = row i.
+__device__ __forceinline__ f32x4 mfma4(h2 a0, h2 a1, h2 b0, h2 b1, f32x4 c) {
+    const h4 a = {a0.x, a0.y, a1.x, a1.y}, b = {b0.x, b0.y, b1.x, b1.y};
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 0, 0, 0);
+}
+
+// The d = 8192 kernels take every sum of products from the matrix cores instead of v_dot2: their
+// waves are bound by vector instructions, four items one after the other (batch 1: 4 of 17 a
+// weight word are dot2; batch 4: 16 of 29), and the matrix cores are idle. Batch 1 and batch
+// 2 .. 4 add in the same order, so a row has the same bits in either. The narrower widths stay
+// with dot2: the staged walk's down tiles hold their sums in registers, four times as many here.
+template <int D>
+constexpr bool kMatrixDots = D >= 8192;
 
 // Waits until every vector memory load this wave issued has returned (s_waitcnt vmcnt(0);
 // expcnt and lgkmcnt at their maxima). The scheduling barriers keep the loads after it
@@ -432,9 +450,38 @@ __device__ __forceinline__ float group_sum(float x) {
 // the nb batch rows (xl: row 0; row b at xl + b N); h of row b goes to hrow + b G.
 // gu_dots adds the dot products of half H of the item (GuHalf) into acc; gu_finish
 // reduces and publishes.
+// A gate/up dot product in progress. With the matrix cores a lane's own product is on the
+// diagonal of its 4x4 block: row l % 4 of A is the lane's x, column l % 4 of B its weights, and
+// its sum is element l % 4 (own). The other twelve are not used; the four lanes need no
+// common columns, so the items' layout is the same.
+template <int D, bool MATRIX = kMatrixDots<D>>
+struct GuSum {
+    float v;
+    __device__ void zero() { v = 0.f; }
+    __device__ void add(const h2 (&w)[4], const uint32_t (&x)[4]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v = dot2(w[q], as_h2(x[q]), v);
+    }
+    __device__ float own() const { return v; }
+};
+template <int D>
+struct GuSum<D, true> {
+    f32x4 v;
+    __device__ void zero() { v = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    __device__ void add(const h2 (&w)[4], const uint32_t (&x)[4]) {
+        v = mfma4(as_h2(x[0]), as_h2(x[1]), w[0], w[1], v);
+        v = mfma4(as_h2(x[2]), as_h2(x[3]), w[2], w[3], v);
+    }
+    __device__ float own() const {
+        const int i = lane_id() & 3;
+        const float lo = i & 1 ? v[1] : v[0], hi = i & 1 ? v[3] : v[2];
+        return i & 2 ? hi : lo;
+    }
+};
+
 template <int D, int NB, int H>
 __device__ __forceinline__ void gu_dots(const GuItem<D>& L, const u32x4* xl, uint32_t nb,
-                                        float (&acc)[NB][GuGeom<D>::RPL][2]) {
+                                        GuSum<D> (&acc)[NB][GuGeom<D>::RPL][2]) {
     using Gm = GuGeom<D>;
     using Hf = GuHalf<D, H>;
     const int r = lane_id() % Gm::LPR;
@@ -465,13 +512,11 @@ __device__ __forceinline__ void gu_dots(const GuItem<D>& L, const u32x4* xl, uin
                     dequant8(words[g], s2, w);
 #pragma unroll
                     for (int b = 0; b < NB; ++b) {
-                        if (NB == 1 || (uint32_t)b < nb) {
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) acc[b][p][proj] = dot2(w[q], as_h2(xw[b][q]), acc[b][p][proj]);
-                        }
+                        if (NB == 1 || (uint32_t)b < nb) acc[b][p][proj].add(w, xw[b]);
                     }
                 }
             }
+            if constexpr (kMatrixDots<D>) __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
@@ -576,10 +621,37 @@ __device__ __forceinline__ bool dn_wait_h(const MlpArgs& a, uint32_t* slot, cons
     return wait_h_word<BACKOFF>(a, slot, hrow, r0, it.h);
 }
 
+// One quarter (columns 8 q .. 8 q + 7 of the lane's 32) of a pass on the matrix cores: sum[c] =
+// the lane's eight rows' products for the batch rows, element i = A's row i, i.e. h of lane
+// i of the four (hw). sw: the scales of the row pairs.
+__device__ __forceinline__ void dn_quarter_products(const DnItem& it, int q, const uint32_t (&sw)[4],
+                                                    const uint32_t (&hw)[4], f32x4 (&sum)[8]) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {   // columns 8 q + 4 half + k
+        h2 w[4][4];                          // [row pair][k]
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+            dequant8(__builtin_amdgcn_perm(it.w[2 * p + 1][q], it.w[2 * p][q], half ? 0x07060302u : 0x05040100u),
+                     as_h2(sw[p]), w[p]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            sum[4 * half + k] = mfma4(as_h2(hw[0]), as_h2(hw[1]), w[0][k], w[1][k], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            sum[4 * half + k] = mfma4(as_h2(hw[2]), as_h2(hw[3]), w[2][k], w[3][k], sum[4 * half + k]);
+    }
+    __builtin_amdgcn_sched_barrier(0);   // one quarter at a time: the kernels are at their register limit
+}
+
 // Adds one pass into the lane's 32 column partials. The pass's h and scales go through
 // this wave's LDS rows (hs: 64 halves; ss: 64 halves per block) so that a lane reads its
 // 8 rows as one 16-byte vector each. Rows (8g + 2p, 8g + 2p + 1) share a dot2: v_perm
 // pairs their nibbles column by column. Rows beyond G have zero weights, h and scales.
+//
+// With MATRIX four lanes that share a row group (8 g + dc, dc in 0..3 or 4..7) are one 4x4 product:
+// A = the eight h (the same in the four lanes), column = the lane's own, two products of four
+// rows each, element 0. The columns go in quarters of 8, so that only their results are held.
+template <bool MATRIX>
 __device__ __forceinline__ void dn_accumulate(const DnItem& it, uint16_t* hs, uint16_t* ss, float acc[32]) {
     const int lane = lane_id(), g = lane >> 3, dc = lane & 7;
     hs[lane] = __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float((uint32_t)it.h));   // exact: h is fp16
@@ -592,6 +664,16 @@ __device__ __forceinline__ void dn_accumulate(const DnItem& it, uint16_t* hs, ui
     const u32x4 sv = *reinterpret_cast<const u32x4*>(ss + kDnRows * (dc >> 2) + 8 * g);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w}, sw[4] = {sv.x, sv.y, sv.z, sv.w};
+    if constexpr (MATRIX) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            f32x4 sum[8];
+            dn_quarter_products(it, q, sw, hw, sum);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) acc[8 * q + c] += sum[c][0];
+        }
+        return;
+    }
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         const u32x4 wa = it.w[2 * p], wb = it.w[2 * p + 1];
@@ -858,7 +940,7 @@ __device__ __forceinline__ float dn_reduce8(const float acc[8]) {
 // each quarter summed over the row groups at once (dn_reduce8): part[r][q] is column
 // 32 dc + 8 q + g of the tile for row r. The dot2 order and the reduction tree are those of
 // dn_accumulate and dn_reduce: every row gets the bits a one-row item would give it.
-template <int NB>
+template <int NB, bool MATRIX>
 __device__ __forceinline__ void dn_accumulate_rows(const DnItem& it, const uint16_t (*hb)[kDnRows], uint16_t* ss,
                                                    uint32_t nb, float (&part)[NB][4]) {
     const int lane = lane_id(), g = lane >> 3, dc = lane & 7;
@@ -868,6 +950,24 @@ __device__ __forceinline__ void dn_accumulate_rows(const DnItem& it, const uint1
     const u32x4 sv = *reinterpret_cast<const u32x4*>(ss + kDnRows * (dc >> 2) + 8 * g);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     const uint32_t sw[4] = {sv.x, sv.y, sv.z, sv.w};
+    if constexpr (MATRIX) {   // row r of A is batch row r: lane l passes h of row l % 4
+        static_assert(NB == 4, "a 4x4 product's rows are the batch rows");
+        const u32x4 hv = *reinterpret_cast<const u32x4*>(&hb[lane & 3][8 * g]);
+        const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            f32x4 sum[8];
+            dn_quarter_products(it, q, sw, hw, sum);
+#pragma unroll
+            for (int r = 0; r < NB; ++r) {
+                float acc[8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c) acc[c] = sum[c][r];
+                if ((uint32_t)r < nb) part[r][q] = dn_reduce8(acc);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {   // columns 8 q + 0..7 of the lane's 32
         float acc[NB][8];
@@ -1301,11 +1401,14 @@ __device__ __forceinline__ bool process_items(const MlpArgs& a, Shared& sh, u32x
     };
     auto compute_gu = [&](uint32_t k, GuItem<D>& gi, const ItemMeta& m) {
         if (a.first_compute && m.n0 == 0 && lane_id() == 0) a.first_compute[m.dest] = now_ticks();
-        float acc[NB][Gm::RPL][2];
+        GuSum<D> acc[NB][Gm::RPL][2];
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int p = 0; p < Gm::RPL; ++p) acc[b][p][0] = acc[b][p][1] = 0.f;
+            for (int p = 0; p < Gm::RPL; ++p) {
+                acc[b][p][0].zero();
+                acc[b][p][1].zero();
+            }
         if constexpr (halves) {
             wait_vector_loads();   // the first half has landed: the second goes out now
             gu_issue<D, 2>(m.grp, m.sc, m.n0, m.nvalid, gi);
@@ -1314,7 +1417,14 @@ __device__ __forceinline__ bool process_items(const MlpArgs& a, Shared& sh, u32x
         } else {
             gu_dots<D, NB, 0>(gi, xl, nb, acc);
         }
-        gu_finish<D, NB>(acc, m.hrow, G, m.n0, m.nvalid, a.seq, nb);
+        float dots[NB][Gm::RPL][2];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int p = 0; p < Gm::RPL; ++p)
+#pragma unroll
+                for (int proj = 0; proj < 2; ++proj) dots[b][p][proj] = acc[b][p][proj].own();
+        gu_finish<D, NB>(dots, m.hrow, G, m.n0, m.nvalid, a.seq, nb);
         if (k == 0) stamp(a, kStampFirstData);
     };
     auto compute_dn = [&](uint32_t k, DnItem& di, const ItemMeta& m) -> bool {
@@ -1341,7 +1451,7 @@ __device__ __forceinline__ bool process_items(const MlpArgs& a, Shared& sh, u32x
                     hb[r][lane] = __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float((uint32_t)hr[r]));   // exact
                 }
                 float part[NB][4];
-                dn_accumulate_rows<NB>(di, hb, ss, nb, part);
+                dn_accumulate_rows<NB, kMatrixDots<D>>(di, hb, ss, nb, part);
                 const int col0 = dn_tile_column(lane);
 #pragma unroll
                 for (int r = 0; r < NB; ++r) {
@@ -1366,12 +1476,12 @@ __device__ __forceinline__ bool process_items(const MlpArgs& a, Shared& sh, u32x
         for (int c = 0; c < 32; ++c) acc[c] = 0.f;
         if constexpr (PACKED) {
             if (!wait_h_lanes(a, slot, pl.hp, di.h)) return false;
-            dn_accumulate(di, hs, ss, acc);
+            dn_accumulate<kMatrixDots<D>>(di, hs, ss, acc);
         } else {
             for (int r0 = 0; r0 < (int)G; r0 += kDnRows) {
                 if (r0) dn_issue<D>(m.grp, m.sc, m.hrow, (int)G, (int)m.tile, r0, a.seq, di);
                 if (!dn_wait_h<NB == 1>(a, slot, m.hrow, (int)G, r0, di)) return false;
-                dn_accumulate(di, hs, ss, acc);
+                dn_accumulate<kMatrixDots<D>>(di, hs, ss, acc);
             }
         }
         float cs[4];
