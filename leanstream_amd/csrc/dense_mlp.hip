@@ -509,6 +509,8 @@ __device__ __forceinline__ void check_dense_queue(const MlpArgs& a, uint32_t* sl
     }
 }
 
+constexpr uint64_t kBlockEndTicks = 200000000;   // 2 s of the 100 MHz clock
+
 struct DenseReduceParams {
     const float* dpart;
     uint32_t width, batch, dsplits;
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
                                                                 MlpArgs args) {
     // the launch's last block (the column blocks are counted from the preloaded arguments)
     if (blockIdx.x == (hot_batch * hot_width / 4 + kThreads - 1) / kThreads) {
-        const MlpArgs a = late_params_as<DenseReduceParams>()->args;
+        MlpArgs a = late_params_as<DenseReduceParams>()->args;
         uint32_t* slot = a.sync + (a.seq & 1) * a.slot_words;
         // The last block only clears the next launch's ring slot (its last user, the previous
         // launch, has finished: stream order) and checks the layer's queue (a read of host
@@ -531,8 +533,17 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
         // launch, with or without core units.
         uint32_t* other = a.sync + ((a.seq + 1) & 1) * a.slot_words;
         for (uint32_t i = threadIdx.x; i < ring_words_used(a); i += blockDim.x) st_agent(other + i, 0u);
-        if (threadIdx.x == 0) check_dense_queue(a, slot);
-        finish_launch(a, slot);
+        if (threadIdx.x < 64) {
+            if (threadIdx.x == 0) check_dense_queue(a, slot);
+            drain_vmem();   // a status bit raised there precedes the completion word
+        }
+        __syncthreads();   // the next ring slot is clear
+        // Then it polls the column blocks' counters, as a fused launch's mirror does: they count
+        // out without waiting for an answer (two returning levels made the launch's end a round
+        // trip longer). The blocks wait for nothing, so the caller's bound for waits on the
+        // host, which may be short, is not theirs.
+        a.spin_limit = max(a.spin_limit, kBlockEndTicks);
+        if (threadIdx.x < 64) await_workers(a, slot, blockIdx.x);
         return;
     }
     // four consecutive columns of one row per thread (width is a multiple of 256): every
@@ -568,7 +579,7 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
                             (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v.w) << 16;
         *reinterpret_cast<u32x2*>(a.y + idx) = u32x2{lo, hi};
     }
-    finish_launch(a, slot);
+    count_out(slot);
 }
 
 namespace {

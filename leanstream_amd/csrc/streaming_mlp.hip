@@ -178,46 +178,6 @@ __device__ __forceinline__ void run_mirror(const MlpArgs& a, uint32_t* slot, uin
     for (uint32_t i = t; i < a.width * a.batch; i += n) st_agent_u64(other_acc + (size_t)i * kAccStride, 0ull);
 }
 
-// Completion proof of a fused launch (replaces a per-launch event). Every worker
-// workgroup counts itself out once its memory operations are complete, with a
-// non-returning atomic into the counter of its group (blk % 8, so no word takes more
-// than an eighth of the increments), and leaves at once. The mirror workgroup, after
-// mirroring the queue, polls the eight counters; when every worker is out it stores the
-// launch sequence into the host-coherent completion word. All reads of the launch's
-// weights and all writes of its outputs are complete by then. (One host store per launch:
-// a sign-off per workgroup into host memory made every launch wait for hundreds of PCIe
-// writes at its end.)
-__device__ __forceinline__ void count_out(uint32_t* slot) {
-    drain_vmem();      // this wave's loads have returned, its stores and atomics are acknowledged
-    __syncthreads();   // every wave of the workgroup has drained
-    if (threadIdx.x == 0)
-        (void)__hip_atomic_fetch_add(slot + kSyncExitGroups + (blockIdx.x % 8u) * kLine, 1u, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void await_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers,
-                                              bool store_done = true) {
-    const uint32_t lane = lane_id();
-    const uint32_t want = lane < 8u ? (workers + 7u - lane) / 8u : 0u;   // workers b < W with b % 8 == lane
-    Waiter wt(a.spin_limit);
-    for (;;) {
-        const uint32_t got = lane < 8u ? ld_agent(slot + kSyncExitGroups + lane * kLine) : 0u;
-        if (__all(got >= want)) break;
-        if (wt.expired()) {   // a worker cannot leave: report it, then complete anyway
-            if (lane == 0) raise_status(a, slot, kStatusTimeout);
-            break;
-        }
-        // about 0.45 us between rounds while any group is less than half out, then at once
-        // (C1 10.28 -> 10.23 us)
-        if (__any(lane < 8u && got * 2u < want))
-            __builtin_amdgcn_s_sleep(16);
-        else
-            __builtin_amdgcn_s_sleep(1);
-    }
-    stamp(a, kStampMirrorDone);
-    if (store_done && lane == 0) __hip_atomic_store(a.done, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // The layer's epilogue in the fused launch's last workgroup (256 threads), once every worker
 // is out: epilogue_kernel's arithmetic on the same y -- each column's fp16 value formed from
 // its accumulator word as the worker that completed it formed it (acc_value), read back at
