@@ -34,9 +34,7 @@ namespace lsamd {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kDenseCols = 256;    // down-projection columns per workgroup: whole 128-byte weight lines
 constexpr int kDenseDnWaves = 8;   // down-projection waves per workgroup: four pairs
-constexpr uint32_t kDenseDnGroups = 256;   // down-projection workgroups: one a CU
 constexpr int kDenseGuWaves = 8;   // gate/up waves per workgroup
 constexpr uint32_t kDenseGuGroups = 256;   // gate/up workgroups: one a CU
 
@@ -383,7 +381,7 @@ __global__ __launch_bounds__(64 * kDenseDnWaves, 2) void dense_down_kernel(const
     const uint32_t D = hot_width, splits = hot_splits;
     const uint32_t lane = lane_id(), w = wave_id(), q = lane >> 4, o = lane & 15;
     // XCD-aware order (workgroup blk runs on XCD blk % 8): consecutive splits go to consecutive
-    // XCDs, so with 8 or 16 splits all tiles of a split, which read the same h rows and scale
+    // XCDs, so with 8, 16 or 32 splits all tiles of a split, which read the same h rows and scale
     // lines, share an L2.
     const uint32_t split = blockIdx.x % splits, tile = blockIdx.x / splits;
     const uint32_t half = w & 1, pair = w >> 1;
@@ -625,8 +623,7 @@ hipError_t launch_dense(const MlpArgs& args, const Bounds& bounds, hipStream_t s
         e = hipLaunchKernel(gu.fn, dim3(groups * halves), dim3(64 * kDenseGuWaves), gargs, 0, stream);
         // One workgroup a CU, and no more splits than leave each pair of its waves a step.
         const uint32_t tiles = a.width / kDenseCols;
-        a.dsplits = std::min({kDenseSplits, std::max(1u, kDenseDnGroups / tiles),
-                              (2 * a.core_count + kDenseDnWaves / 2 - 1) / (kDenseDnWaves / 2)});
+        a.dsplits = std::min(dense_splits(a.width), (2 * a.core_count + kDenseDnWaves / 2 - 1) / (kDenseDnWaves / 2));
         void* dargs[] = {&a.core, &a.core_count, &a.width, &a.dsplits, &a, &b};
         const void* down = a.batch > 16 ? reinterpret_cast<const void*>(&dense_down_kernel<2>)
                                         : reinterpret_cast<const void*>(&dense_down_kernel<1>);

@@ -116,7 +116,7 @@ int HipBackend::bind(const HipLayerBuffers& b) {
     if (e == hipSuccess && dense)
         e = hipMalloc(&p.h16, sizeof(uint16_t) * 32 * b.slot_capacity * b.group_size);
     if (e == hipSuccess && dense)
-        e = hipMalloc(&p.dpart, sizeof(float) * lsamd::kDenseSplits * 32 * b.width);
+        e = hipMalloc(&p.dpart, sizeof(float) * lsamd::dense_splits(b.width) * 32 * b.width);
     // h rows >= batch stay zero: the dense down projection reads all 32 rows
     if (e == hipSuccess && dense) e = hipMemset(p.h16, 0, sizeof(uint16_t) * 32 * b.slot_capacity * b.group_size);
     if (e == hipSuccess)
@@ -189,7 +189,7 @@ int HipBackend::bind(const HipLayerBuffers& b) {
     a.slot_capacity = b.slot_capacity;
     a.h16 = p.h16;
     a.dpart = p.dpart;
-    a.dsplits = dense ? lsamd::kDenseSplits : 0u;
+    a.dsplits = dense ? lsamd::dense_splits(b.width) : 0u;
     p.bounds = {b.cache_groups, b.staging_groups, b.physical_groups};
     slices_ = b.width / lsamd::kDnCols;
     max_workers_ = static_cast<uint32_t>(p.cus * p.per_cu_fused) - 1;

@@ -1,8 +1,9 @@
 // Device building blocks of the gfx950 streaming sparse INT4 MLP kernels, shared by the
-// per-layer persistent kernels (streaming_mlp.hip) and the multi-layer chain kernel
-// (chain_mlp.hip): memory helpers, exact INT4 dequantisation, gate/up and down-projection
-// items (register and LDS-staged walks), the deterministic fixed-point column reduction,
-// descriptor access and validation, and the ready-queue mirror and claim protocol.
+// per-layer persistent kernels (streaming_mlp.hip), the multi-layer chain kernel
+// (chain_mlp.hip) and the dense batched kernels (dense_mlp.hip): memory helpers, exact INT4
+// dequantisation, gate/up and down-projection items (register and LDS-staged walks), the
+// deterministic fixed-point column reduction, descriptor access and validation, the
+// ready-queue mirror and claim protocol, and the launches' ends.
 // Everything here is inline device code; kernels and host code live in the .hip files.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -141,8 +142,9 @@ __device__ __forceinline__ f32x4 mfma4(h2 a0, h2 a1, h2 b0, h2 b1, f32x4 c) {
 // The d = 8192 kernels take every sum of products from the matrix cores instead of v_dot2: their
 // waves are bound by vector instructions, four items one after the other (batch 1: 4 of 17 a
 // weight word are dot2; batch 4: 16 of 29), and the matrix cores are idle. Batch 1 and batch
-// 2 .. 4 add in the same order, so a row has the same bits in either. The narrower widths stay
-// with dot2: the staged walk's down tiles hold their sums in registers, four times as many here.
+// 2 .. 4 add in the same order, so a row has the same bits in either. Four layers of 90 groups:
+// one row 96.4 -> 94.4 us, four rows 206.0 -> 195.7. The narrower widths stay with dot2: the
+// staged walk's down tiles hold their sums in registers, four times as many here.
 template <int D>
 constexpr bool kMatrixDots = D >= 8192;
 
