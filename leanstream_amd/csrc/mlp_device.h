@@ -139,12 +139,17 @@ __device__ __forceinline__ f32x4 mfma4(h2 a0, h2 a1, h2 b0, h2 b1, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 0, 0, 0);
 }
 
-// The d = 8192 kernels take every sum of products from the matrix cores instead of v_dot2: their
-// waves are bound by vector instructions, four items one after the other (batch 1: 4 of 17 a
-// weight word are dot2; batch 4: 16 of 29), and the matrix cores are idle. Batch 1 and batch
-// 2 .. 4 add in the same order, so a row has the same bits in either. Four layers of 90 groups:
-// one row 96.4 -> 94.4 us, four rows 206.0 -> 195.7. The narrower widths stay with dot2: the
-// staged walk's down tiles hold their sums in registers, four times as many here.
+// The d = 8192 kernels take their gate/up sums from the matrix cores instead of v_dot2: their
+// waves are bound by vector instructions, four items one after the other, of which dot2 is 4 of
+// 17 a gate/up weight word at batch 1 and 16 of 29 at batch 4, and the matrix cores are idle.
+// Batch 1 and batch 2 .. 4 add in the same order, so a row has the same bits in either. Four
+// layers of 90 groups, one to four rows: 101.9, 148.8, 176.7, 206.8 -> 101.7, 144.6, 168.5,
+// 194.1 us; through the split entry point 103.4, 156.8, 186.7, 219.1 -> 102.3, 152.3, 178.6,
+// 206.4. The down items stay with dot2: as 4x4 products they spilled the batch 2 .. 4 kernels
+// (34 registers, 116 bytes of scratch; none with dot2) and computed four rows whatever the batch:
+// 147.4, 173.2, 196.9 us at two to four rows, and 78.7 against 72.8 for two rows of 20 groups.
+// The narrower widths stay with dot2: the staged walk's down tiles hold their sums in
+// registers.
 template <int D>
 constexpr bool kMatrixDots = D >= 8192;
 
@@ -623,37 +628,10 @@ __device__ __forceinline__ bool dn_wait_h(const MlpArgs& a, uint32_t* slot, cons
     return wait_h_word<BACKOFF>(a, slot, hrow, r0, it.h);
 }
 
-// One quarter (columns 8 q .. 8 q + 7 of the lane's 32) of a pass on the matrix cores: sum[c] =
-// the lane's eight rows' products for the batch rows, element i = A's row i, i.e. h of lane
-// i of the four (hw). sw: the scales of the row pairs.
-__device__ __forceinline__ void dn_quarter_products(const DnItem& it, int q, const uint32_t (&sw)[4],
-                                                    const uint32_t (&hw)[4], f32x4 (&sum)[8]) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {   // columns 8 q + 4 half + k
-        h2 w[4][4];                          // [row pair][k]
-#pragma unroll
-        for (int p = 0; p < 4; ++p)
-            dequant8(__builtin_amdgcn_perm(it.w[2 * p + 1][q], it.w[2 * p][q], half ? 0x07060302u : 0x05040100u),
-                     as_h2(sw[p]), w[p]);
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            sum[4 * half + k] = mfma4(as_h2(hw[0]), as_h2(hw[1]), w[0][k], w[1][k], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            sum[4 * half + k] = mfma4(as_h2(hw[2]), as_h2(hw[3]), w[2][k], w[3][k], sum[4 * half + k]);
-    }
-    __builtin_amdgcn_sched_barrier(0);   // one quarter at a time: the kernels are at their register limit
-}
-
 // Adds one pass into the lane's 32 column partials. The pass's h and scales go through
 // this wave's LDS rows (hs: 64 halves; ss: 64 halves per block) so that a lane reads its
 // 8 rows as one 16-byte vector each. Rows (8g + 2p, 8g + 2p + 1) share a dot2: v_perm
 // pairs their nibbles column by column. Rows beyond G have zero weights, h and scales.
-//
-// With MATRIX four lanes that share a row group (8 g + dc, dc in 0..3 or 4..7) are one 4x4 product:
-// A = the eight h (the same in the four lanes), column = the lane's own, two products of four
-// rows each, element 0. The columns go in quarters of 8, so that only their results are held.
-template <bool MATRIX>
 __device__ __forceinline__ void dn_accumulate(const DnItem& it, uint16_t* hs, uint16_t* ss, float acc[32]) {
     const int lane = lane_id(), g = lane >> 3, dc = lane & 7;
     hs[lane] = __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float((uint32_t)it.h));   // exact: h is fp16
@@ -666,16 +644,6 @@ __device__ __forceinline__ void dn_accumulate(const DnItem& it, uint16_t* hs, ui
     const u32x4 sv = *reinterpret_cast<const u32x4*>(ss + kDnRows * (dc >> 2) + 8 * g);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w}, sw[4] = {sv.x, sv.y, sv.z, sv.w};
-    if constexpr (MATRIX) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            f32x4 sum[8];
-            dn_quarter_products(it, q, sw, hw, sum);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) acc[8 * q + c] += sum[c][0];
-        }
-        return;
-    }
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         const u32x4 wa = it.w[2 * p], wb = it.w[2 * p + 1];
@@ -942,7 +910,7 @@ __device__ __forceinline__ float dn_reduce8(const float acc[8]) {
 // each quarter summed over the row groups at once (dn_reduce8): part[r][q] is column
 // 32 dc + 8 q + g of the tile for row r. The dot2 order and the reduction tree are those of
 // dn_accumulate and dn_reduce: every row gets the bits a one-row item would give it.
-template <int NB, bool MATRIX>
+template <int NB>
 __device__ __forceinline__ void dn_accumulate_rows(const DnItem& it, const uint16_t (*hb)[kDnRows], uint16_t* ss,
                                                    uint32_t nb, float (&part)[NB][4]) {
     const int lane = lane_id(), g = lane >> 3, dc = lane & 7;
@@ -952,24 +920,6 @@ __device__ __forceinline__ void dn_accumulate_rows(const DnItem& it, const uint1
     const u32x4 sv = *reinterpret_cast<const u32x4*>(ss + kDnRows * (dc >> 2) + 8 * g);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     const uint32_t sw[4] = {sv.x, sv.y, sv.z, sv.w};
-    if constexpr (MATRIX) {   // row r of A is batch row r: lane l passes h of row l % 4
-        static_assert(NB == 4, "a 4x4 product's rows are the batch rows");
-        const u32x4 hv = *reinterpret_cast<const u32x4*>(&hb[lane & 3][8 * g]);
-        const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            f32x4 sum[8];
-            dn_quarter_products(it, q, sw, hw, sum);
-#pragma unroll
-            for (int r = 0; r < NB; ++r) {
-                float acc[8];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) acc[c] = sum[c][r];
-                if ((uint32_t)r < nb) part[r][q] = dn_reduce8(acc);
-            }
-        }
-        return;
-    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {   // columns 8 q + 0..7 of the lane's 32
         float acc[NB][8];
@@ -1453,7 +1403,7 @@ __device__ __forceinline__ bool process_items(const MlpArgs& a, Shared& sh, u32x
                     hb[r][lane] = __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float((uint32_t)hr[r]));   // exact
                 }
                 float part[NB][4];
-                dn_accumulate_rows<NB, kMatrixDots<D>>(di, hb, ss, nb, part);
+                dn_accumulate_rows<NB>(di, hb, ss, nb, part);
                 const int col0 = dn_tile_column(lane);
 #pragma unroll
                 for (int r = 0; r < NB; ++r) {
@@ -1478,12 +1428,12 @@ __device__ __forceinline__ bool process_items(const MlpArgs& a, Shared& sh, u32x
         for (int c = 0; c < 32; ++c) acc[c] = 0.f;
         if constexpr (PACKED) {
             if (!wait_h_lanes(a, slot, pl.hp, di.h)) return false;
-            dn_accumulate<kMatrixDots<D>>(di, hs, ss, acc);
+            dn_accumulate(di, hs, ss, acc);
         } else {
             for (int r0 = 0; r0 < (int)G; r0 += kDnRows) {
                 if (r0) dn_issue<D>(m.grp, m.sc, m.hrow, (int)G, (int)m.tile, r0, a.seq, di);
                 if (!dn_wait_h<NB == 1>(a, slot, m.hrow, (int)G, r0, di)) return false;
-                dn_accumulate<kMatrixDots<D>>(di, hs, ss, acc);
+                dn_accumulate(di, hs, ss, acc);
             }
         }
         float cs[4];

@@ -29,13 +29,16 @@ CASES = [(512, 5, 1), (512, 17, 3), (512, 16, 37),             # two items a wor
          (8192, 16, 2), (8192, 17, 1), (8192, 32, 21)]
 
 
-def dense(torch, d, batch, units, bad=()):
-    """A core-only dense launch over random groups; returns (y32, per-row oracle inputs, status)."""
+def dense(torch, d, batch, units, bad=(), row=None, table=None):
+    """A core-only launch over random groups; returns (y32, per-row oracle inputs, status). With
+    `row`, a launch of that row of the batch alone; `table`: an offline kernel table."""
     gen = torch.Generator().manual_seed(d + 64 * batch + units)
     gb, sw = 64 * 3 * d // 2, 64 * 3 * (d // 128)
     cache = torch.randint(0, 256, (units * gb,), dtype=torch.uint8, generator=gen)
     scales = (torch.rand(units * sw, generator=gen) * 0.015 + 0.005).half()
-    x = torch.randn(batch, d, generator=gen).to(torch.bfloat16)
+    x = torch.randn(batch, d, generator=gen).to(torch.bfloat16 if batch > 4 else torch.float16)
+    if row is not None:
+        x, batch = x[row:row + 1], 1
     slots = torch.randperm(units, generator=gen).numpy()
     rows = np.zeros((units, 5), dtype=np.uint32)
     rows[:, 0] = rows[:, 1] = rows[:, 2] = slots
@@ -46,7 +49,7 @@ def dense(torch, d, batch, units, bad=()):
     dev = [t.cuda() for t in (cache, scales, x)]
     y = torch.full((batch, d), float("nan"), dtype=torch.float16, device="cuda")
     y32 = torch.full((batch, d), float("nan"), dtype=torch.float32, device="cuda")
-    backend, queue = NativeBackend(), ReadyQueue(1)
+    backend, queue = NativeBackend(table), ReadyQueue(1)
     try:
         backend.bind(d, 64, units, dev[0], dev[1], physical_groups=units, cache_groups=units, queue_capacity=1,
                      batch=batch, y32=y32)
@@ -111,3 +114,18 @@ def test_matrix_products_at_other_groups(torch_gpu, G, batch):
         check_rows(layer, layer.core_rows[0], cfg.name)
     finally:
         layer.close()
+
+
+@pytest.mark.parametrize("entry,table", [("fused", None), ("split", [[4]])])
+@pytest.mark.parametrize("batch", [2, 3, 4])
+def test_batch_rows_have_the_one_row_bits(torch_gpu, batch, entry, table):
+    """d = 8192, 64-neuron groups: two and three rows take the kernels of four, and every row gets
+    the bits of a launch of its own through either entry point."""
+    print(f"case: d=8192 batch={batch} {entry} against one row at a time", flush=True)
+    y32, inputs, status = dense(torch_gpu, 8192, batch, 13, table=table)
+    assert status == 0, status
+    check(y32, inputs, inputs[0], f"d8192 b{batch} {entry}")
+    for row in range(batch):
+        one, _, status = dense(torch_gpu, 8192, batch, 13, row=row)
+        assert status == 0, status
+        assert np.array_equal(one[0].view(np.uint32), y32[row].view(np.uint32)), row
