@@ -78,7 +78,10 @@ struct HipLayerBuffers {
     uint32_t* claim_log = nullptr;      // optional claim log: 4 words per range a workgroup takes
                                         // ({first, count, ready at claim or ~0u, worker}), in the order
                                         // taken; holds queue_capacity ranges
-    uint64_t* stamps = nullptr;         // optional per-worker phase stamps [max workers][32]
+    uint64_t* stamps = nullptr;         // optional phase stamps, a row of 32 per wave of batch-1..4 launches:
+                                        // [12 * compute units][32] (three workgroups of four waves a
+                                        // compute unit is the most the split entry point runs, the fused
+                                        // one runs two); dense launches write none
 };
 
 // Optional layer epilogue, run after every enqueue on the same stream (no LeanStream

@@ -61,7 +61,7 @@ typedef struct ls_hip_layer_buffers {
     uint32_t* executions;
     uint64_t* first_compute;
     uint32_t* claim_log;      /* optional: 4 words per range taken, queue_capacity ranges */
-    uint64_t* stamps;
+    uint64_t* stamps;         /* optional: [12 * compute units][32] (leanstream/hip_backend.h) */
 } ls_hip_layer_buffers;
 
 /* Consumer modes (leanstream::runtime::ConsumerMode). */

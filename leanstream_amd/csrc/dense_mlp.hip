@@ -541,7 +541,10 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
         // trip longer). The blocks wait for nothing, so the caller's bound for waits on the
         // host, which may be short, is not theirs.
         a.spin_limit = max(a.spin_limit, kBlockEndTicks);
-        if (threadIdx.x < 64) await_workers(a, slot, blockIdx.x);
+        if (threadIdx.x < 64) {
+            if (!poll_workers(a, slot, blockIdx.x) && threadIdx.x == 0) raise_status(a, slot, kStatusTimeout);
+            store_done(a);
+        }
         return;
     }
     // four consecutive columns of one row per thread (width is a multiple of 256): every

@@ -72,6 +72,7 @@ constexpr uint32_t kClaimStatic = 0xFFFFFFFFu;
 // Phase stamps (100 MHz clock) written by lane 0 of every wave when MlpArgs::stamps is
 // set: stamps[(block * 4 + wave) * kStampSlots + phase]; 0 = the wave never got there.
 constexpr uint32_t kStampSlots = 32;
+constexpr int kStampWgPerCu = 3;   // most workgroups a CU of a stamped grid: sizes a caller's rows
 enum StampPhase : uint32_t {
     kStampEntry = 0,
     kStampDescs = 1,         // the wave's first descriptors have arrived
@@ -200,7 +201,7 @@ struct MlpArgs {
     uint32_t* done;               // host-coherent: the last workgroup of a launch stores seq
     uint32_t* claim_log;          // optional: kClaimLogWords words per claimed range, in claim order
     uint32_t claim_log_cap;       // entries (ranges) claim_log holds
-    uint64_t* stamps;             // optional: per-worker phase stamps [workers][kStampSlots] (100 MHz clock)
+    uint64_t* stamps;             // optional: phase stamps [grid * 4][kStampSlots] (100 MHz clock)
     // geometry / control
     uint32_t width;               // d
     uint32_t group_size;          // G

@@ -2173,18 +2173,15 @@ __device__ __forceinline__ void count_out(uint32_t* slot) {
                                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ void await_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers,
-                                              bool store_done = true) {
+// True once workgroups 0 .. workers - 1 have counted out, false when the bound has passed. One wave.
+__device__ __forceinline__ bool poll_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers) {
     const uint32_t lane = lane_id();
     const uint32_t want = lane < 8u ? (workers + 7u - lane) / 8u : 0u;   // workers b < W with b % 8 == lane
     Waiter wt(a.spin_limit);
     for (;;) {
         const uint32_t got = lane < 8u ? ld_agent(slot + kSyncExitGroups + lane * kLine) : 0u;
-        if (__all(got >= want)) break;
-        if (wt.expired()) {   // a worker cannot leave: report it, then complete anyway
-            if (lane == 0) raise_status(a, slot, kStatusTimeout);
-            break;
-        }
+        if (__all(got >= want)) return true;
+        if (wt.expired()) return false;
         // about 0.45 us between rounds while any group is less than half out, then at once
         // (C1 10.28 -> 10.23 us)
         if (__any(lane < 8u && got * 2u < want))
@@ -2192,8 +2189,19 @@ __device__ __forceinline__ void await_workers(const MlpArgs& a, uint32_t* slot, 
         else
             __builtin_amdgcn_s_sleep(1);
     }
+}
+
+__device__ __forceinline__ void store_done(const MlpArgs& a) {
+    if (lane_id() == 0) __hip_atomic_store(a.done, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The mirror's wave at the end of a fused launch.
+__device__ __forceinline__ void await_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers,
+                                              bool complete = true) {
+    // a worker cannot leave: report it, then complete anyway
+    if (!poll_workers(a, slot, workers) && lane_id() == 0) raise_status(a, slot, kStatusTimeout);
     stamp(a, kStampMirrorDone);
-    if (store_done && lane == 0) __hip_atomic_store(a.done, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (complete) store_done(a);
 }
 
 // Completion proof of the split launch sequence, at the end of its last kernel (the

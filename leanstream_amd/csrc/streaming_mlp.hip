@@ -37,6 +37,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <algorithm>
 #include "mlp_args.h"
 #include "mlp_launch.h"
 
@@ -504,7 +505,7 @@ hipError_t resident_workers(int width, int entry_point, int batch, int group_siz
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&na, v->stage_a[nb], kThreads, 0);
         if (na < n) n = na;
     }
-    *per_cu = n;
+    *per_cu = std::min(n, kStampWgPerCu);
     return e;
 }
 

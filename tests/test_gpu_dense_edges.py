@@ -99,6 +99,20 @@ def test_dense_bad_descriptor_is_reported_and_left_out(torch_gpu, d, batch):
     check(y32, inputs, np.delete(inputs[0], (2, 8), axis=0), f"d{d} b{batch} without the rejected units")
 
 
+def test_dense_launch_writes_no_stamps(torch_gpu):
+    """Stamp rows are the waves of a batch-1..4 grid; a dense launch's grids are larger."""
+    cfg = config(1024, batch=5, dense=True)
+    print(f"case: stamps bound to {cfg.name}", flush=True)
+    layer = DeviceLayer(cfg, stamps=True)
+    try:
+        layer.seal_empty_queue(1)
+        layer.run_core(epoch=1)
+        sync_and_check_status(torch_gpu, layer)
+        assert not layer.stamps.any().item()
+    finally:
+        layer.close()
+
+
 @pytest.mark.parametrize("G,batch", [(128, 1), (8, 1), (16, 3), (128, 2)])
 def test_matrix_products_at_other_groups(torch_gpu, G, batch):
     """d = 8192: the plain walk's two-pass down tiles, the packed walk, a pass of fewer than 64 rows
