@@ -507,7 +507,32 @@ __device__ __forceinline__ void check_dense_queue(const MlpArgs& a, uint32_t* sl
     }
 }
 
-constexpr uint64_t kBlockEndTicks = 200000000;   // 2 s of the 100 MHz clock
+// Completion of a dense launch: the word is stored once every column block has counted out, by one
+// wave, whatever the bound on waits. The last block polls the counters, as a fused launch's mirror
+// does (the blocks count out without waiting for an answer: two returning levels made the
+// launch's end a round trip longer). When its bound passes first -- column blocks that wait for a
+// CU behind another stream's kernel -- it leaves the launch's sequence in kSyncExit: a
+// block that has counted out looks there, and the one that finds every block out stores the
+// word. The poller leaves the sequence before its own last look and a block counts before its own
+// (each acknowledged), so one of them sees the other; whoever takes the sequence out stores.
+__device__ __forceinline__ void take_over(const MlpArgs& a, uint32_t* slot, uint32_t blocks) {
+    bool half;
+    uint32_t seq = a.seq;
+    if (workers_out(slot, blocks, half) && lane_id() == 0 &&
+        __hip_atomic_compare_exchange_strong(glb(slot + kSyncExit), &seq, 0u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+        store_done(a);
+}
+
+__device__ __forceinline__ void await_blocks(const MlpArgs& a, uint32_t* slot, uint32_t blocks) {
+    if (a.spin_limit && poll_workers(a, slot, blocks)) {
+        store_done(a);
+        return;
+    }
+    if (lane_id() == 0) st_agent(slot + kSyncExit, a.seq);
+    drain_vmem();
+    take_over(a, slot, blocks);
+}
 
 struct DenseReduceParams {
     const float* dpart;
@@ -523,7 +548,7 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
                                                                 MlpArgs args) {
     // the launch's last block (the column blocks are counted from the preloaded arguments)
     if (blockIdx.x == (hot_batch * hot_width / 4 + kThreads - 1) / kThreads) {
-        MlpArgs a = late_params_as<DenseReduceParams>()->args;
+        const MlpArgs a = late_params_as<DenseReduceParams>()->args;
         uint32_t* slot = a.sync + (a.seq & 1) * a.slot_words;
         // The last block only clears the next launch's ring slot (its last user, the previous
         // launch, has finished: stream order) and checks the layer's queue (a read of host
@@ -536,15 +561,7 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
             drain_vmem();   // a status bit raised there precedes the completion word
         }
         __syncthreads();   // the next ring slot is clear
-        // Then it polls the column blocks' counters, as a fused launch's mirror does: they count
-        // out without waiting for an answer (two returning levels made the launch's end a round
-        // trip longer). The blocks wait for nothing, so the caller's bound for waits on the
-        // host, which may be short, is not theirs.
-        a.spin_limit = max(a.spin_limit, kBlockEndTicks);
-        if (threadIdx.x < 64) {
-            if (!poll_workers(a, slot, blockIdx.x) && threadIdx.x == 0) raise_status(a, slot, kStatusTimeout);
-            store_done(a);
-        }
+        if (threadIdx.x < 64) await_blocks(a, slot, blockIdx.x);
         return;
     }
     // four consecutive columns of one row per thread (width is a multiple of 256): every
@@ -581,6 +598,10 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(const float* hot
         *reinterpret_cast<u32x2*>(a.y + idx) = u32x2{lo, hi};
     }
     count_out(slot);
+    if (threadIdx.x < 64) {
+        drain_vmem();   // counted
+        if (ld_agent(slot + kSyncExit) == a.seq) take_over(a, slot, gridDim.x - 1);
+    }
 }
 
 namespace {

@@ -15,7 +15,8 @@ using leanstream::runtime::QueueControl;
 // its own 128-byte line.
 constexpr uint32_t kLine = 32;  // 32-bit words per 128-byte line
 enum SyncWord : uint32_t {
-    kSyncExit = 0 * kLine,        // groups of workgroups (kSyncExitGroups) that have finished
+    kSyncExit = 0 * kLine,        // groups of workgroups (kSyncExitGroups) that have finished; dense
+                                  // launch: its sequence once the last block no longer polls
     kSyncEpoch = 1 * kLine,       // mirror: state | path << 2 | total << 4 (state 0 unseen, 1 ok, 2 leave)
     kSyncReady = 2 * kLine,       // mirror: published positions copied into qmirror
     kSyncClaimHead = 3 * kLine,   // next unclaimed ready position (claim path)

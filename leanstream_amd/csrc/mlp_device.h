@@ -2173,18 +2173,24 @@ __device__ __forceinline__ void count_out(uint32_t* slot) {
                                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// True once workgroups 0 .. workers - 1 have counted out, false when the bound has passed. One wave.
-__device__ __forceinline__ bool poll_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers) {
+// Have workgroups 0 .. workers - 1 counted out? `half`: is any group less than half out? One wave.
+__device__ __forceinline__ bool workers_out(uint32_t* slot, uint32_t workers, bool& half) {
     const uint32_t lane = lane_id();
     const uint32_t want = lane < 8u ? (workers + 7u - lane) / 8u : 0u;   // workers b < W with b % 8 == lane
+    const uint32_t got = lane < 8u ? ld_agent(slot + kSyncExitGroups + lane * kLine) : 0u;
+    half = __any(lane < 8u && got * 2u < want);
+    return __all(got >= want);
+}
+
+// True once they have, false when the bound has passed.
+__device__ __forceinline__ bool poll_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers) {
     Waiter wt(a.spin_limit);
-    for (;;) {
-        const uint32_t got = lane < 8u ? ld_agent(slot + kSyncExitGroups + lane * kLine) : 0u;
-        if (__all(got >= want)) return true;
+    for (bool half;;) {
+        if (workers_out(slot, workers, half)) return true;
         if (wt.expired()) return false;
         // about 0.45 us between rounds while any group is less than half out, then at once
         // (C1 10.28 -> 10.23 us)
-        if (__any(lane < 8u && got * 2u < want))
+        if (half)
             __builtin_amdgcn_s_sleep(16);
         else
             __builtin_amdgcn_s_sleep(1);

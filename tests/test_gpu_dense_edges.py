@@ -8,6 +8,8 @@ more items a workgroup, which are taken in batches), 16 and 17 batch rows (one a
 fragments; at d = 8192 the second 16 rows go to workgroups of their own), every width's split of
 the columns over waves, and down splits with idle waves.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -109,6 +111,35 @@ def test_dense_launch_writes_no_stamps(torch_gpu):
         layer.run_core(epoch=1)
         sync_and_check_status(torch_gpu, layer)
         assert not layer.stamps.any().item()
+    finally:
+        layer.close()
+
+
+@pytest.mark.parametrize("d,batch,units", [(512, 5, 1), (1024, 16, 0), (8192, 32, 9)])
+def test_dense_completion_without_the_poll(torch_gpu, d, batch, units):
+    """With a bound of zero the reduction's last block does not poll: the word still comes, after the
+    outputs, no status bit is raised, and the outputs are those of a launch that polls."""
+    torch = torch_gpu
+    print(f"case: completion handed over, dense d={d} batch={batch} units={units}", flush=True)
+    cfg = config(d, batch=batch, dense=True)
+    layer = DeviceLayer(cfg)
+    try:
+        layer.seal_empty_queue(1)
+        layer.k = min(units, layer.k)
+        layer.run_core(epoch=1)
+        sync_and_check_status(torch, layer)
+        want = layer.y32.clone()
+        layer.backend.set_spin_limit(0)
+        for _ in range(50):   # both ring slots; the poller or a column block ends the launch
+            layer.y32.fill_(float("nan"))
+            torch.cuda.synchronize()
+            layer.run_core(epoch=1)
+            deadline = time.monotonic() + 10
+            while not layer.backend.complete():
+                assert time.monotonic() < deadline
+            got = layer.y32.clone()
+            sync_and_check_status(torch, layer)
+            assert torch.equal(got.view(torch.int32), want.view(torch.int32))
     finally:
         layer.close()
 
