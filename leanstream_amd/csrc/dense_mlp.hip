@@ -645,7 +645,8 @@ hipError_t launch_dense(const MlpArgs& args, const Bounds& bounds, hipStream_t s
         uint32_t halves = gu.halves;
         void* gargs[] = {&a.core, &a.x, &a.core_count, &a.batch, &groups, &halves, &a, &b};
         e = hipLaunchKernel(gu.fn, dim3(groups * halves), dim3(64 * kDenseGuWaves), gargs, 0, stream);
-        // One workgroup a CU, and no more splits than leave each pair of its waves a step.
+        // One workgroup a CU, and a split for every four steps, one a wave pair (rounded up: a
+        // small layer's pairs may be idle, no split is).
         const uint32_t tiles = a.width / kDenseCols;
         a.dsplits = std::min(dense_splits(a.width), (2 * a.core_count + kDenseDnWaves / 2 - 1) / (kDenseDnWaves / 2));
         void* dargs[] = {&a.core, &a.core_count, &a.width, &a.dsplits, &a, &b};

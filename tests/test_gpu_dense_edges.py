@@ -3,10 +3,11 @@ their splits can go wrong, against the CPU oracle (relative L2 <= 1e-3, max-abs 
 fp32 output, as for the other widths: fp16 roundings of g, u, silu and h that a sum in another
 order moves by a unit in the last place).
 
-Dense: gate/up items of 8 neurons and their rounds (one unit; fewer items than workgroups; 64 and
-more items a workgroup, which are taken in batches), 16 and 17 batch rows (one and two MFMA row
-fragments; at d = 8192 the second 16 rows go to workgroups of their own), every width's split of
-the columns over waves, and down splits with idle waves.
+Dense: gate/up items of 8 neurons and their rounds (one unit; fewer items than workgroups; more than
+64 items a workgroup or down steps a wave, which are taken in batches of 64), 16 and 17 batch rows
+(one and two MFMA row fragments; at d = 8192 the second 16 rows go to workgroups of their own),
+every width's split of the columns over waves, and down splits with idle waves. d = 8192 at batch
+1 .. 4: group sizes of every walk, and every row of a batch against a launch of that row alone.
 """
 import time
 
@@ -25,10 +26,11 @@ REL_L2, MAX_ABS = 1e-3, 2e-2   # max-abs of outputs of root mean square up to 1;
 STATUS_BAD_DESCRIPTOR = 4
 
 CASES = [(512, 5, 1), (512, 17, 3), (512, 16, 37),             # two items a workgroup at a time
-         (1024, 16, 1), (1024, 17, 33), (1024, 5, 2049),       # 64 and more items and steps a workgroup
+         (1024, 16, 1), (1024, 17, 33), (1024, 5, 2049),       # more than 64 items a workgroup, two a round
          (2048, 7, 5), (2048, 16, 67), (2048, 17, 3),
          (4096, 6, 1), (4096, 16, 9), (4096, 17, 33), (4096, 31, 40),
-         (8192, 16, 2), (8192, 17, 1), (8192, 32, 21)]
+         (8192, 16, 2), (8192, 17, 1), (8192, 32, 21),
+         (8192, 17, 1100)]   # more than 64 items a workgroup, one a round, and more than 64 steps a down wave
 
 
 def dense(torch, d, batch, units, bad=(), row=None, table=None):

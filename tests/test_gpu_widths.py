@@ -77,7 +77,7 @@ def test_core_layer_at_every_width(torch_gpu, d, G, batch):
 
 @pytest.mark.parametrize("d,batch", [(512, 32), (2048, 32), (1024, 5), (1024, 19)])
 def test_dense_layer_at_other_widths(torch_gpu, d, batch):
-    """Other widths, and batches below 32 (rows >= batch of x16 and h16 are zero)."""
+    """Other widths, and batches below 32 (x rows past the batch repeat the last one, h16 rows are zero)."""
     torch = torch_gpu
     cfg = config(d, batch=batch, dense=True)
     log(f"case: dense layer {cfg.name} k={cfg.active}")
