@@ -303,10 +303,11 @@ struct WeightManager::Impl {
             m.queue.fail(EINVAL);
             return;
         }
-        // before finalize there is no plan: finalize publishes what is READY by then
-        if (!m.is_frozen()) return;
+        // Before finalize there is no plan: finalize publishes what is READY by then. The phase is
+        // read under finalize's lock: without it this read may pass the group's READY store, and
+        // finalize's read of READY its own store of the phase, so that neither publishes.
         std::lock_guard<std::mutex> lock(m.producer);
-        if (m.current(c.epoch)) m.publish_member(c.logical_group, c.staging_slot);
+        if (m.current(c.epoch) && m.is_frozen()) m.publish_member(c.logical_group, c.staging_slot);
     }
 };
 
