@@ -516,16 +516,20 @@ __device__ __forceinline__ void check_dense_queue(const MlpArgs& a, uint32_t* sl
 // word. The poller leaves the sequence before its own last look and a block counts before its own
 // (each acknowledged), so one of them sees the other; whoever takes the sequence out stores.
 __device__ __forceinline__ void take_over(const MlpArgs& a, uint32_t* slot, uint32_t blocks) {
-    bool half;
+    const uint32_t lane = lane_id();
+    const uint32_t want = lane < 8u ? (blocks + 7u - lane) / 8u : 0u;   // blocks b with b % 8 == lane
+    const uint32_t got = lane < 8u ? ld_agent(slot + kSyncExitGroups + lane * kLine) : 0u;
     uint32_t seq = a.seq;
-    if (workers_out(slot, blocks, half) && lane_id() == 0 &&
+    if (__all(got >= want) && lane == 0 &&
         __hip_atomic_compare_exchange_strong(glb(slot + kSyncExit), &seq, 0u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT))
         store_done(a);
 }
 
 __device__ __forceinline__ void await_blocks(const MlpArgs& a, uint32_t* slot, uint32_t blocks) {
-    if (a.spin_limit && poll_workers(a, slot, blocks)) {
+    bool out = a.spin_limit != 0;
+    if (out) poll_workers(a, slot, blocks, [&] { out = false; });
+    if (out) {
         store_done(a);
         return;
     }

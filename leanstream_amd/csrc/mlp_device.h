@@ -2173,24 +2173,23 @@ __device__ __forceinline__ void count_out(uint32_t* slot) {
                                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Have workgroups 0 .. workers - 1 counted out? `half`: is any group less than half out? One wave.
-__device__ __forceinline__ bool workers_out(uint32_t* slot, uint32_t workers, bool& half) {
+// One wave waits until workgroups 0 .. workers - 1 have counted out; calls `expired` and leaves once
+// the bound has passed.
+template <class Expired>
+__device__ __forceinline__ void poll_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers, Expired expired) {
     const uint32_t lane = lane_id();
     const uint32_t want = lane < 8u ? (workers + 7u - lane) / 8u : 0u;   // workers b < W with b % 8 == lane
-    const uint32_t got = lane < 8u ? ld_agent(slot + kSyncExitGroups + lane * kLine) : 0u;
-    half = __any(lane < 8u && got * 2u < want);
-    return __all(got >= want);
-}
-
-// True once they have, false when the bound has passed.
-__device__ __forceinline__ bool poll_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers) {
     Waiter wt(a.spin_limit);
-    for (bool half;;) {
-        if (workers_out(slot, workers, half)) return true;
-        if (wt.expired()) return false;
+    for (;;) {
+        const uint32_t got = lane < 8u ? ld_agent(slot + kSyncExitGroups + lane * kLine) : 0u;
+        if (__all(got >= want)) break;
+        if (wt.expired()) {
+            expired();
+            break;
+        }
         // about 0.45 us between rounds while any group is less than half out, then at once
         // (C1 10.28 -> 10.23 us)
-        if (half)
+        if (__any(lane < 8u && got * 2u < want))
             __builtin_amdgcn_s_sleep(16);
         else
             __builtin_amdgcn_s_sleep(1);
@@ -2204,8 +2203,9 @@ __device__ __forceinline__ void store_done(const MlpArgs& a) {
 // The mirror's wave at the end of a fused launch.
 __device__ __forceinline__ void await_workers(const MlpArgs& a, uint32_t* slot, uint32_t workers,
                                               bool complete = true) {
-    // a worker cannot leave: report it, then complete anyway
-    if (!poll_workers(a, slot, workers) && lane_id() == 0) raise_status(a, slot, kStatusTimeout);
+    poll_workers(a, slot, workers, [&] {   // a worker cannot leave: report it, then complete anyway
+        if (lane_id() == 0) raise_status(a, slot, kStatusTimeout);
+    });
     stamp(a, kStampMirrorDone);
     if (complete) store_done(a);
 }
