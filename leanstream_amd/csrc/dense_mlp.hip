@@ -128,9 +128,10 @@ __device__ __forceinline__ uint64_t lane_pointer(uint64_t v, uint32_t lane) {
 // 4096 x 224 groups, twice the weights) by a launch of its own. The weight loads of the
 // next round (two items; one at d >= 4096, whose items are four steps and more) are in flight
 // while a round is computed. At the end of a round the waves' partial tiles meet in LDS in a
-// fixed order, one barrier a round: two items a round and no loads past the end took the kernel
-// from 7.1 to 5.9 us at 2048 columns x 128 groups x 7 rows; at 4096 x 224 x 32 one item a round
-// is the better (17.6 us, two 18.5).
+// fixed order, one barrier a round. Two items a round are the better up to d = 2048, one above (a
+// layer at 7 and 32 rows, two items against one: 1024 columns x 128 groups 15.9 and 18.5 us
+// against 16.5 and 18.6, 2048 x 128 equal, 4096 x 224 32.7 and 39.6 against 32.2 and 38.4, 8192 x
+// 90 30.3 and 39.6 against 28.8 and 37.4; 16 and 17 rows alike).
 //
 // Where the x of 17 .. 32 rows does not fit the registers (d = 8192) a workgroup takes 16 rows
 // (`halves` = 2): workgroups blk and blk + 8, on one XCD, read the same weights.
