@@ -450,13 +450,6 @@ __device__ __forceinline__ float group_sum(float x) {
     return x;
 }
 
-// Finish a gate/up item: dot products, row reductions, activation. Publishes h of
-// neurons n0 .. n0 + nvalid - 1 into hrow, each word tagged with the launch sequence
-// (the word is its own ready flag).
-// With NB > 1 the item's weights are dequantised once and multiplied with x of each of
-// the nb batch rows (xl: row 0; row b at xl + b N); h of row b goes to hrow + b G.
-// gu_dots adds the dot products of half H of the item (GuHalf) into acc; gu_finish
-// reduces and publishes.
 // A gate/up dot product in progress. With the matrix cores a lane's own product is on the
 // diagonal of its 4x4 block: row l % 4 of A is the lane's x, column l % 4 of B its weights, and
 // its sum is element l % 4 (own). The other twelve are not used; the four lanes need no
@@ -486,6 +479,13 @@ struct GuSum<D, true> {
     }
 };
 
+// Finish a gate/up item: dot products, row reductions, activation. Publishes h of
+// neurons n0 .. n0 + nvalid - 1 into hrow, each word tagged with the launch sequence
+// (the word is its own ready flag).
+// With NB > 1 the item's weights are dequantised once and multiplied with x of each of
+// the nb batch rows (xl: row 0; row b at xl + b N); h of row b goes to hrow + b G.
+// gu_dots adds the dot products of half H of the item (GuHalf) into acc; gu_finish
+// reduces and publishes.
 template <int D, int NB, int H>
 __device__ __forceinline__ void gu_dots(const GuItem<D>& L, const u32x4* xl, uint32_t nb,
                                         GuSum<D> (&acc)[NB][GuGeom<D>::RPL][2]) {
